@@ -68,6 +68,7 @@ _OTHER = {
     "helm_paged_attn_noalloc_max_floats": ([], _i64),
     "helm_argmax_workspace_bytes": ([_i32], _i64),
     "helm_int8_gemv_workspace_bytes": ([_i32, _i32, _i32], _i64),
+    "helm_int8_gemv_split_bytes": ([_i32, _i32, _i32], _i64),
 }
 
 

@@ -694,11 +694,27 @@ static int int8_gemv_impl(const void* x, int64_t ldx, const void* norm_w, float 
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.kt = choose_kt(M, K);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // 3-16 tokens: the matrix-core small-M kernel where it takes the shape (with a
-  // norm prologue at K = 4096; measured faster than the streaming kernel at 3-4
-  // tokens too)
-  if (helm::launch_int8_small_m(x, ldx, norm_w, eps, q, ldq, scale, bias, residual, y, ldy, M, N,
-                                K, part, part_bytes, s)) {
+  // 3-16 tokens, two matrix-core forms.  One 16-row tile per workgroup with x^T in
+  // LDS (gemv_small_m.hip) where its grid is whole and x fits: K = 4096 (4096 ->
+  // 12288 at 16 tokens 12.2 against 14.9 us, 4096 -> 4096 7.4 against 9.2), and K of
+  // 6145-16384 whose row tiles fill the 256 CUs in one round (12288 -> 4096 at 8
+  // tokens 14.8 against 16.8 us; at 8-16 tokens only as its split form).  Elsewhere
+  // x^T in registers, persistent over the row tiles (gemv_xreg.hip): 17408 -> 5120
+  // at 8 tokens 34.4 -> 23.9 us, 12288 -> 5120 20.5 -> 17.4, 5120 -> 17408 29.6 ->
+  // 19.9, 6144 -> 4096 13.6 -> 10.5.
+  const int tiles = (N + 15) / 16;
+  const bool tile_form = K == 4096 || (K > 6144 && K <= 16384 && tiles > 224 && tiles <= 256 &&
+                                       (M < 8 || K % 3072 == 0));
+  auto tile = [&] {
+    return helm::launch_int8_small_m(x, ldx, norm_w, eps, q, ldq, scale, bias, residual, y, ldy, M, N,
+                                     K, part, part_bytes, s);
+  };
+  auto xreg = [&] {
+    return helm::launch_xreg_int8(x, ldx, norm_w, eps, q, ldq, scale, bias, residual, y, ldy, M, N, K,
+                                  part, part_bytes, s);
+  };
+  // (a call without the workspace long K needs, or unaligned, falls to the other)
+  if (tile_form ? (tile() || xreg()) : (xreg() || tile())) {
     HELM_CHECK_LAUNCH("helm_int8_gemv launch");
     return HELM_OK;
   }
@@ -725,6 +741,10 @@ extern "C" int64_t helm_int8_gemv_workspace_bytes(int M, int N, int K) {
   return helm::int8_small_m_workspace_bytes(M, N, K);
 }
 
+extern "C" int64_t helm_int8_gemv_split_bytes(int M, int N, int K) {
+  return std::max(helm::int8_small_m_workspace_bytes(M, N, K), helm::xreg_workspace_bytes(M, N, K));
+}
+
 extern "C" int helm_int8_gemv_ws(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
                                  const void* scale, const void* bias, const void* residual,
                                  void* y, int64_t ldy, int M, int N, int K, void* workspace,
@@ -737,7 +757,7 @@ extern "C" int helm_int8_gemv_ws(const void* x, int64_t ldx, const int8_t* q, in
     HELM_CHECK_ARG(helm::aligned16(workspace), "helm_int8_gemv_ws: workspace must be 16-byte aligned");
   }
   return int8_gemv_impl(x, ldx, nullptr, 0.f, q, ldq, scale, bias, residual, y, ldy, M, N, K,
-                        need > 0 ? static_cast<float*>(workspace) : nullptr, workspace_bytes, stream);
+                        static_cast<float*>(workspace), workspace ? workspace_bytes : 0, stream);
 }
 
 extern "C" int helm_int8_gemv(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
@@ -745,6 +765,18 @@ extern "C" int helm_int8_gemv(const void* x, int64_t ldx, const int8_t* q, int64
                               int M, int N, int K, void* stream) {
   return helm_int8_gemv_fused(x, ldx, nullptr, 0.f, q, ldq, scale, bias, nullptr, y, ldy, M, N, K,
                               stream);
+}
+
+// fp16 weights at 3-16 tokens on the matrix cores; false when neither form takes
+// the shape.  x^T in registers from K = 2048 on (4096 -> 151936 at 4 / 16 tokens 233
+// -> 195 and 246 -> 211 us; 5120 at 16 tokens, whose x rows exceed LDS, 1058 -> 260),
+// x^T in LDS below (1024 -> 151936 at 8 tokens 54.4 against 55.4 us).
+static bool fp16_matrix_form(const void* x, int64_t ldx, const void* norm_w, float eps,
+                             const void* w, int64_t ldw, const void* bias, void* y, int64_t ldy,
+                             int M, int N, int K, hipStream_t s) {
+  auto lds = [&] { return helm::launch_fp16_small_m(x, ldx, norm_w, eps, w, ldw, bias, y, ldy, M, N, K, s); };
+  auto xreg = [&] { return helm::launch_xreg_fp16(x, ldx, norm_w, eps, w, ldw, bias, y, ldy, M, N, K, s); };
+  return K < 2048 ? (lds() || xreg()) : (xreg() || lds());
 }
 
 extern "C" int helm_fp16_gemv(const void* x, int64_t ldx, const void* w, int64_t ldw,
@@ -759,7 +791,7 @@ extern "C" int helm_fp16_gemv(const void* x, int64_t ldx, const void* w, int64_t
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.kt = choose_kt(M, K);
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!helm::launch_fp16_small_m(x, ldx, nullptr, 0.f, w, ldw, bias, y, ldy, M, N, K, s))
+  if (!fp16_matrix_form(x, ldx, nullptr, 0.f, w, ldw, bias, y, ldy, M, N, K, s))
     launch_m<false, EPI_PLAIN, false>(a, s);
   HELM_CHECK_LAUNCH("helm_fp16_gemv launch");
   return HELM_OK;
@@ -779,7 +811,7 @@ extern "C" int helm_fp16_gemv_rmsnorm(const void* x, int64_t ldx, const void* no
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.kt = choose_kt(M, K);
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!helm::launch_fp16_small_m(x, ldx, norm_w, eps, w, ldw, nullptr, y, ldy, M, N, K, s))
+  if (!fp16_matrix_form(x, ldx, norm_w, eps, w, ldw, nullptr, y, ldy, M, N, K, s))
     launch_m<false, EPI_PLAIN, true>(a, s);
   HELM_CHECK_LAUNCH("helm_fp16_gemv_rmsnorm launch");
   return HELM_OK;
@@ -802,9 +834,12 @@ extern "C" int helm_int8_gemv_swiglu(const void* x, int64_t ldx, const void* nor
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.kt = choose_kt(M, K);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // 3-16 tokens at K = 4096: norm, gate and up on the matrix cores in one launch
+  // 3-16 tokens: norm, gate and up on the matrix cores in one launch, K = 4096 with
+  // x^T in LDS (4096 -> 2 x 12288 at 8 tokens 21.4 against 24.1 us), any other K up
+  // to 6144 with x^T in registers (5120 -> 2 x 17408 at 12 tokens 345 -> 38 us)
   if (helm::launch_int8_small_m_swiglu(x, ldx, norm_w, eps, q_gate, s_gate, q_up, s_up, ldq, y, ldy,
-                                       M, N, K, s)) {
+                                       M, N, K, s) ||
+      helm::launch_xreg_swiglu(x, ldx, norm_w, eps, q_gate, s_gate, q_up, s_up, ldq, y, ldy, M, N, K, s)) {
     HELM_CHECK_LAUNCH("helm_int8_gemv_swiglu launch");
     return HELM_OK;
   }

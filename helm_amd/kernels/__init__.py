@@ -107,7 +107,7 @@ def int8_linear(input: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
         return out
     stream = _native.stream_ptr(input.device)
     if M <= GEMV_MAX_TOKENS:
-        ws_bytes = gemv_workspace_bytes(M, N, K)
+        ws_bytes = gemv_split_bytes(M, N, K)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=input.device) if ws_bytes else None
         _native.call("helm_int8_gemv_ws", x2.data_ptr(), x2.stride(0), qweight.data_ptr(),
                      qweight.stride(0), scale.data_ptr(), _native.ptr(bias), None, y2.data_ptr(),
@@ -120,9 +120,16 @@ def int8_linear(input: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
 
 @functools.lru_cache(maxsize=None)
 def gemv_workspace_bytes(M: int, N: int, K: int) -> int:
-    """Workspace helm_int8_gemv_ws uses at this shape (0: none): the split-K
+    """Workspace helm_int8_gemv_ws requires at this shape (0: none): the split-K
     form's fp32 partial sums for 8-16 tokens over long K."""
     return int(_native.lib().helm_int8_gemv_workspace_bytes(int(M), int(N), int(K)))
+
+
+@functools.lru_cache(maxsize=None)
+def gemv_split_bytes(M: int, N: int, K: int) -> int:
+    """Workspace with which helm_int8_gemv_ws takes its fastest form at this shape
+    (0: none; at least gemv_workspace_bytes)."""
+    return int(_native.lib().helm_int8_gemv_split_bytes(int(M), int(N), int(K)))
 
 
 def fp16_linear(input: torch.Tensor, weight: torch.Tensor,

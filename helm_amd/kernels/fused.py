@@ -13,7 +13,7 @@ from typing import Optional
 import torch
 
 from .. import _native
-from . import gemv_workspace_bytes
+from . import gemv_split_bytes
 
 
 def _check_fp16(*ts):
@@ -81,7 +81,7 @@ def int8_gemv_fused(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
             res = y2.data_ptr()
     if norm_weight is None:
         # no norm prologue: the workspace form (split K for long K at 5-16 tokens)
-        ws_bytes = gemv_workspace_bytes(M, N, K)
+        ws_bytes = gemv_split_bytes(M, N, K)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
         _native.call("helm_int8_gemv_ws", x2.data_ptr(), x2.stride(0), qweight.data_ptr(),
                      qweight.stride(0), scale.data_ptr(), _native.ptr(bias), res, y2.data_ptr(),

@@ -104,7 +104,7 @@ class BatchDecodeEngine:
         self.act = torch.empty(B, sh.ffn, dtype=torch.float16, device=dev)
         self.logits = torch.empty(B, sh.vocab, dtype=torch.float16, device=dev)
         self.argmax_ws = fused.argmax_workspace(B, dev)
-        self.gemv_ws_bytes = hk.gemv_workspace_bytes(B, sh.hidden, sh.ffn)
+        self.gemv_ws_bytes = hk.gemv_split_bytes(B, sh.hidden, sh.ffn)
         self.gemv_ws = torch.empty(max(self.gemv_ws_bytes, 16), dtype=torch.uint8, device=dev)
         # step parameters: positions[B], seq_lens[B], slots[L][B], offsets[L][B]
         self.params = torch.zeros(2 * B + 2 * sh.n_layers * B, dtype=torch.int32, device=dev)

@@ -95,6 +95,10 @@ int helm_int8_gemv_fused(const void* x, int64_t ldx, const void* norm_w, float e
  * up to the fp32 summation order.  Replaces the same decode fast path as
  * helm_int8_gemv (helm/kernels/fp16_gemv.cpp:105-157). */
 int64_t helm_int8_gemv_workspace_bytes(int M, int N, int K);
+/* Bytes with which helm_int8_gemv_ws takes its fastest form (0: no workspace
+ * helps; never below helm_int8_gemv_workspace_bytes): fp32 partial sums of k
+ * slices for 3-16 tokens over K beyond one workgroup's registers. */
+int64_t helm_int8_gemv_split_bytes(int M, int N, int K);
 int helm_int8_gemv_ws(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
                       const void* scale, const void* bias, const void* residual,
                       void* y, int64_t ldy, int M, int N, int K,

@@ -565,3 +565,56 @@ def test_fp16_module_patch_and_disable_flag(monkeypatch):
         y32 = seq[0](x)
         ref32 = torch.nn.functional.linear(x.float(), w0.float(), seq[0].bias.float()).half()
         assert torch.equal(y32, ref32)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 16, 16), (3, 1, 144), (16, 1001, 1040), (5, 4113, 2048), (8, 33, 5104),
+                                   (16, 5120, 6144), (12, 4099, 6160), (9, 270, 17360), (16, 8200, 12304),
+                                   (7, 512, 25600)])
+def test_x_in_registers_int8(M, N, K):
+    """The 3-16 token kernel with x^T in registers: K that ends inside a 128-byte
+    unit or leaves waves without one, the largest K of one k slice (6144) and the
+    first past it, odd N, one row tile, several per workgroup; plain with bias,
+    residual aliasing y, SwiGLU, and the same through rows with a stride."""
+    g = np.random.default_rng(K + N + M)
+    x, q, s, b = make_inputs(M, N, K, seed=K + 3 * N + M, bias=True)
+    _, q2, s2, _ = make_inputs(M, N, K, seed=K + 5 * N + M)
+    res = g.standard_normal((M, N)).astype(np.float16)
+    xd, qd, sd, bd, resd, q2d, s2d = to_dev(x, q, s, b, res, q2, s2)
+    lin = ol.int8_linear_exact(x, q, s, b)
+    bound = accumulation_bound(x, q, s)
+    assert_linear_ok(hk.int8_linear(xd, qd, sd, bd).cpu().numpy(), lin, f"M={M} N={N} K={K}", bound)
+    wide = torch.full((M, K + 8), float("nan"), dtype=torch.float16, device="cuda")
+    wide[:, :K] = xd
+    assert_linear_ok(hk.int8_linear(wide[:, :K], qd, sd, bd).cpu().numpy(), lin, "strided x", bound)
+    y = resd.clone()
+    fused.int8_gemv_fused(xd, qd, sd, bias=bd, residual=y, out=y)
+    exp = res.astype(np.float64) + lin.astype(np.float16).astype(np.float64)
+    slack = ulp16(lin) + bound + ulp16(exp)
+    assert (np.abs(y.cpu().numpy().astype(np.float64) - exp) <= slack).all()
+    if K > 6144:      # SwiGLU beyond one k slice takes the kernel it took before
+        return
+    a = fused.int8_gemv_swiglu(xd, qd, sd, q2d, s2d).cpu().numpy()
+    gt, up = (ol.int8_linear_exact(x, *w).astype(np.float16).astype(np.float64) for w in ((q, s), (q2, s2)))
+    assert swiglu_within_bar(a, gt, up)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 31, 2048), (16, 1000, 2112), (5, 70000, 2048), (16, 515, 5120), (4, 40, 6144)])
+def test_x_in_registers_fp16(M, N, K):
+    """fp16 weights with x^T in registers: K whose units do not divide by the
+    waves, more row tiles than one round, odd N, bias; an infinite weight reaches
+    its own output only."""
+    g = torch.Generator(device="cuda").manual_seed(K + N + M)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.05).half()
+    b = torch.randn(N, generator=g, device="cuda").half()
+    w[N // 2, K - 1] = float("inf")
+    x[:, K - 1] = 1.0
+    y = hk.fp16_linear(x, w, b).double().cpu()
+    exact = x.double().cpu() @ w.double().cpu().t() + b.double().cpu()
+    assert torch.isinf(y[:, N // 2]).all() and (y[:, N // 2] > 0).all()
+    keep = torch.arange(N) != N // 2
+    # fp32 accumulation (2^-22 of the summed magnitudes) and one rounding to fp16
+    wk = w.double().cpu().abs()
+    wk[N // 2] = 0
+    bound = (x.double().cpu().abs() @ wk.t()) * 2.0 ** -22 + exact.nan_to_num(0, 0, 0).abs() * 2.0 ** -11 + 2.0 ** -24
+    assert ((y - exact).abs() <= bound)[:, keep].all()
