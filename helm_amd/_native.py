@@ -42,6 +42,8 @@ _SIGNATURES = {
                                   _f32, _vp],
     "helm_prefill_attn": [_vp, _i64, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _f32,
                           _vp, _i64, _i64, _vp],
+    "helm_prefill_attn_ws": [_vp, _i64, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _f32,
+                          _vp, _i64, _i64, _vp, _i64, _vp],
     "helm_prefill_attn_mask": [_vp, _i64, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32,
                                _f32, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp],
     "helm_paged_attn_reduce": [_vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp],
@@ -67,6 +69,7 @@ _OTHER = {
     "helm_paged_attn_max_split_pages": ([], _i32),
     "helm_paged_attn_noalloc_max_floats": ([], _i64),
     "helm_argmax_workspace_bytes": ([_i32], _i64),
+    "helm_prefill_attn_workspace_bytes": ([_i32, _i32, _i32, _i32, _i32], _i64),
     "helm_int8_gemv_workspace_bytes": ([_i32, _i32, _i32], _i64),
     "helm_int8_gemv_split_bytes": ([_i32, _i32, _i32], _i64),
 }

@@ -12,14 +12,23 @@
 // permuted so that each lane holds the probabilities of exactly the 8
 // consecutive keys whose V^T it feeds to the second MFMA.
 //
-// A workgroup is one query head x a block of 4 * 16 * NC queries, one wave per
-// 16 * NC queries.  The four waves need the same K/V tiles, so the workgroup
+// A workgroup is one kv head x a block of 4 * 16 * NC rows, one wave per 16 * NC
+// of them; rows are (query, head of the group) pairs, query-major, so a few
+// queries fill a block with all their heads (17 queries of a group of 4: one
+// block, not four) and a block spans fewer positions of the diagonal.  The four waves need the same K/V tiles, so the workgroup
 // fetches each 32-key tile once, straight into LDS (global_load_lds_dwordx4:
 // every lane moves 16 bytes, a wave 1 KiB of contiguous pool memory), double
 // buffered: tile s+1 is copied while tile s is computed, and the waves read
-// their MFMA operands from LDS.  The copy of tile s+1 is issued only after the
-// operand reads of tile s (the compiler makes LDS reads wait for outstanding
-// copies, so this order keeps the copy in flight across the whole step).  LDS layouts (16-byte chunks) are chosen so
+// their MFMA operands from LDS.  The copy of tile s+1 goes out right after the
+// barrier of step s, from page slots looked up a step earlier, ahead of the operand
+// reads of tile s (a compiler-tracked copy would make those reads wait for it).
+// A step is a serial chain of about 2000 cycles (operand reads, QK, softmax, PV);
+// 64 KB of LDS operand reads per step, 512 cycles of MFMA per wave and about as many of VALU
+// work bound it, two workgroups per CU overlap.  Measured: 14B heads at T =
+// 2048 74.5 -> 67.1 us (641 TFLOP/s), 32 heads, 390 queries over 7000 cached keys
+// (104 workgroups, five key splits) 198 -> 84 us, T = 4096 over 12000 keys 1305 -> 1221 us
+// (966 TFLOP/s), left-padding mask at T = 2048 171 -> 151 us.
+// LDS layouts (16-byte chunks) are chosen so
 // that both the copies and the operand reads are conflict free:
 //   K: row-major [32 keys][D/8 chunks], chunk index XOR-swizzled by key bits
 //      {0,1,3,4}, so the 16 rows one operand read touches hit 16 distinct banks;
@@ -31,6 +40,7 @@
 // each XCD serves one kv head and its K/V stays in that XCD's L2.  fp32 online
 // softmax per query in the log2 domain; keys past the query's position are
 // masked; blocks with the most keys are launched first.
+#include <algorithm>
 #include <type_traits>
 
 #include "helm_common.h"
@@ -71,6 +81,11 @@ struct PrefillArgs {
   // optional per query row t: keys from key_end[t] on are -inf in every head's
   // mask, so a wave (workgroup) stops at the last key step any of its rows sees
   const int32_t* key_end;
+  // SPLIT form: key splits and their fp32 partials, part_o [T, Hq, S, D] (not
+  // normalised) and part_ml [T, Hq, S, 2] (running maximum, sum)
+  int S;
+  float* part_o;
+  float* part_ml;
 };
 
 // Workgroup barrier for the K/V stages: this wave's copies into LDS have landed
@@ -88,11 +103,23 @@ __device__ __forceinline__ h8_t ld_h8_nt(const uint16_t* p) {
   return __builtin_bit_cast(h8_t, __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p)));
 }
 
+// One wave's 1 KiB global -> LDS copy: lane l moves 16 bytes from `src` to LDS
+// byte lds + 16 l.  Inline assembly, so that the compiler does not make the step's
+// operand reads wait for the copies of the next one; the step's barrier waits.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is named as clobbered on purpose
+__device__ __forceinline__ void copy_to_lds(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+               :
+               : "s"(__builtin_amdgcn_readfirstlane(lds)), "v"(src)
+               : "memory", "m0");
+}
+#pragma clang diagnostic pop
+
 template <int D>
 struct KStep {
   h8_t k[2][D / 32];
   h8_t v[D / 16];
-  bool page_ok;     // the page of this lane's 8 keys is valid
 };
 
 // XOR swizzle of K chunk columns: key row r -> bits {0,1} and {3,4} of r, so the
@@ -106,7 +133,7 @@ __device__ __forceinline__ int kswz(int r) {
 // NC: 16-query column tiles per wave; a workgroup covers QB = 64 * NC queries.
 // MASK: every query sees keys 0 .. kv_len - 1 with the additive mask added to its
 // scaled scores (the reference's SDPA with attn_mask); otherwise causal.
-template <int D, int P, int NC, bool MASK>
+template <int D, int P, int NC, bool MASK, bool SPLIT>
 #ifndef PF_WPE
 #define PF_WPE 2
 #endif
@@ -127,19 +154,27 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   __shared__ __attribute__((aligned(16))) u32x4_t s_kv[kNS][kKC + kVC];
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int col = lane & 15;
   const int grp = lane >> 4;
   const int G = a.Hq / a.Hkv;
-  const int nqb = (a.T + kQB - 1) / kQB;
+  const int R = a.T * G;                           // rows (query, head of the group) of a kv head
+  const int nqb = (R + kQB - 1) / kQB;
   const int hk = (int)blockIdx.x % a.Hkv;
   const int r = (int)blockIdx.x / a.Hkv;
-  const int h = hk * G + r % G;
-  const int q0 = (nqb - 1 - r / G) * kQB;         // heaviest (latest) blocks first
-  const int qw = q0 + wave * kWQ;                  // this wave's first query
+  const int sp = SPLIT ? r % a.S : 0;
+  const int q0 = (nqb - 1 - (SPLIT ? r / a.S : r)) * kQB;   // heaviest (latest) blocks first
+  const int qw = q0 + wave * kWQ;                  // this wave's first row
+  int tq[NC], hq[NC];                              // query and head of this lane's columns
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int row = min(qw + c * 16 + col, R - 1);
+    tq[c] = row / G;
+    hq[c] = hk * G + (row - tq[c] * G);
+  }
 
-  const int wg_key_end = MASK ? a.kv_len : a.q_start + min(q0 + kQB, a.T);
+  const int wg_key_end = MASK ? a.kv_len : a.q_start + (min(q0 + kQB, R) - 1) / G + 1;
   const int npages = (wg_key_end + P - 1) / P;
   if (tid == 0) {
     s_bad = 0;
@@ -156,34 +191,29 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   h8_t qb_op[NC][KT];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int qi = min(qw + c * 16 + col, a.T - 1);
 #pragma unroll
     for (int kk = 0; kk < KT; ++kk)
-      qb_op[c][kk] = ld_h8_nt(a.q + (int64_t)qi * a.q_st + (int64_t)h * a.q_sh + kk * 32 + grp * 8);
+      qb_op[c][kk] = ld_h8_nt(a.q + (int64_t)tq[c] * a.q_st + (int64_t)hq[c] * a.q_sh + kk * 32 + grp * 8);
   }
   // MASK: keys [0, w_hi) hold every key some query of this wave can see
   int w_hi = a.kv_len;
   if constexpr (MASK) {
     if (a.key_end) {
       w_hi = 0;
-      for (int i = lane; i < kWQ; i += 64) {
-        const int t = qw + i;
-        if (t < a.T) w_hi = max(w_hi, a.key_end[t]);
-      }
+      for (int t = qw / G + lane; t <= (min(qw + kWQ, R) - 1) / G; t += 64) w_hi = max(w_hi, a.key_end[t]);
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) w_hi = max(w_hi, __shfl_xor(w_hi, off, 64));
       // wave-uniform after the butterfly: held in a scalar register
       w_hi = __builtin_amdgcn_readfirstlane(min(w_hi, a.kv_len));
     }
-    if (qw >= a.T) w_hi = 0;
+    if (qw >= R) w_hi = 0;
     if (lane == 0) atomicMax(&s_kr, w_hi);
   }
   __syncthreads();
 
   // keys [0, key_end) can be seen by some query of this wave
-  const int key_end = qw < a.T ? (MASK ? w_hi : a.q_start + min(qw + kWQ, a.T)) : 0;
+  const int key_end = qw < R ? (MASK ? w_hi : a.q_start + (min(qw + kWQ, R) - 1) / G + 1) : 0;
   const int nsteps = (key_end + kKS - 1) / kKS;
-  // the workgroup's steps [step0, wg_steps)
   // the workgroup's steps [0, wg_steps): with MASK up to the last key any of its
   // rows sees (an LDS value, uniform over the workgroup).  Steps below a row's
   // first visible key are visited anyway (their keys are -inf for it): a loop
@@ -192,7 +222,7 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
                             : (wg_key_end + kKS - 1) / kKS;
   // steps whose keys every query of the wave sees (all below the diagonal, valid
   // pages): no masking
-  const int nfull = (s_bad || MASK) ? 0 : min(nsteps, (a.q_start + qw + 1) / kKS);
+  const int nfull = (s_bad || MASK) ? 0 : min(nsteps, (a.q_start + qw / G + 1) / kKS);
   const int p_last = max(npages - 1, 0);
   const uint16_t* kbase = a.k + (int64_t)hk * a.k_hs;
   const uint16_t* vbase = a.v + (int64_t)hk * a.v_hs;
@@ -223,22 +253,29 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
       c_off[i] = dim * (int)a.v_ds + row % P;
     }
   }
+  // page slots of this thread's chunks of step st: looked up a step ahead, so the
+  // copies go out at once after a step's barrier, ahead of its operand reads
+  int c_slot[kIssue];
+  auto slots = [&](int st) {
+#pragma unroll
+    for (int i = 0; i < kIssue; ++i) c_slot[i] = s_slot[min((st * kKS + c_row[i]) / P, p_last)];
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)&s_kv[0][0];
   auto issue = [&](int st, int b) {
-    const int tok0 = st * kKS;
-    const int in0 = kStepOnPage ? 0 : tok0 % P;       // the step's start inside its page
+    const int in0 = kStepOnPage ? 0 : (st * kKS) % P;  // the step's start inside its page
 #pragma unroll
     for (int i = 0; i < kIssue; ++i) {
       const bool is_k = i * 256 < kKC;                // compile-time per i
-      const int slot = max(s_slot[min((tok0 + c_row[i]) / P, p_last)], 0);
+      const int slot = max(c_slot[i], 0);
       const uint16_t* src =
           is_k ? kbase + (int64_t)slot * a.k_ss + c_off[i] + in0 * D
                : vbase + (int64_t)slot * a.v_ss + c_off[i] + in0;
-      __builtin_amdgcn_global_load_lds(src, (lds_void_t*)&s_kv[b][i * 256 + wave * 64], 16, 0, 0);
+      copy_to_lds(src, lds0 + (uint32_t)((b * (kKC + kVC) + i * 256 + wave * 64) * 16));
     }
   };
 
-  // MFMA operands of key tile s (in stage b), and the validity of its page
-  auto read = [&](KStep<D>& bf, int s, int b) {
+  // MFMA operands of the key tile in stage b
+  auto read = [&](KStep<D>& bf, int b) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int row = (col >> 2) * 8 + t * 4 + (col & 3);
@@ -248,8 +285,6 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
     }
 #pragma unroll
     for (int d = 0; d < DT; ++d) bf.v[d] = __builtin_bit_cast(h8_t, s_kv[b][kKC + d * 64 + grp * 16 + col]);
-    const int tv = s * kKS + grp * 8;
-    bf.page_ok = s_slot[min(tv / P, p_last)] >= 0 && tv / P < npages;
   };
 
   float m_run[NC], l_run[NC];
@@ -273,8 +308,9 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
     constexpr bool FULL = decltype(full_tag)::value;
     const int tok0 = s * kKS;
     const int tv = tok0 + grp * 8;                     // this lane's 8 keys tv .. tv+7
-    const bool page_ok = bf.page_ok;
+    bool page_ok = true;                               // their page is valid
     if constexpr (!FULL) {
+      page_ok = s_slot[min(tv / P, p_last)] >= 0 && tv / P < npages;
       const int nvis = page_ok ? max(0, min(8, key_end - tv)) : 0;
       uint32_t vmask[4];
 #pragma unroll
@@ -290,6 +326,10 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
         bf.v[d] = __builtin_bit_cast(h8_t, vw);
       }
     }
+    // Phases over all column tiles, so that the tiles' MFMA chains interleave: the
+    // scores of every tile, one branch for the rare rescale, the exponentials,
+    // then every tile's PV products.
+    float sv[NC][8];                                   // raw scores of keys tv .. tv+7
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
       f4_t sc0 = {0.f, 0.f, 0.f, 0.f}, sc1 = {0.f, 0.f, 0.f, 0.f};
@@ -298,97 +338,184 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
         sc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf.k[0][kk], qb_op[c][kk], sc0, 0, 0, 0);
         sc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf.k[1][kk], qb_op[c][kk], sc1, 0, 0, 0);
       }
-      float sv[8];                                     // raw scores of keys tv .. tv+7
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        sv[r] = sc0[r];
-        sv[4 + r] = sc1[r];
+        sv[c][r] = sc0[r];
+        sv[c][4 + r] = sc1[r];
       }
+    }
+    float mx[NC];
+    bool raise = false;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
       if constexpr (MASK) {
         // mask of this lane's query row at keys tv .. tv+7 (loaded after the score
         // MFMAs: fewer registers live across them); scores are scaled at the
         // exponent, so the mask enters divided by the scale
-        const int qm = min(qw + c * 16 + col, a.T - 1);
         const u32x4_t mraw =
-            *reinterpret_cast<const u32x4_t*>(a.mask + (int64_t)h * a.m_sh + (int64_t)qm * a.m_si + tv);
+            *reinterpret_cast<const u32x4_t*>(a.mask + (int64_t)hq[c] * a.m_sh + (int64_t)tq[c] * a.m_si + tv);
         const h8_t mh = __builtin_bit_cast(h8_t, mraw);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sv[j] = __builtin_fmaf((float)mh[j], a.inv_scale, sv[j]);
+        for (int j = 0; j < 8; ++j) sv[c][j] = __builtin_fmaf((float)mh[j], a.inv_scale, sv[c][j]);
       }
       if constexpr (!FULL) {
-        const int qi = qw + c * 16 + col;              // query index of this lane's column
-        // keys visible to this query: tv + j <= q_start + qi, or < kv_len with a mask
-        // (and inside valid pages)
-        const int kend = MASK ? a.kv_len : a.q_start + qi + 1;
-        const int nvalid = (page_ok && qi < a.T) ? max(0, min(8, kend - tv)) : 0;
+        // keys visible to this row's query: tv + j <= its position, or < kv_len with
+        // a mask (and inside valid pages)
+        const int kend = MASK ? a.kv_len : a.q_start + tq[c] + 1;
+        const int nvalid = (page_ok && qw + c * 16 + col < R) ? max(0, min(8, kend - tv)) : 0;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) sv[j] = j < nvalid ? sv[j] : -INFINITY;
+        for (int j = 0; j < 8; ++j) sv[c][j] = j < nvalid ? sv[c][j] : -INFINITY;
       }
       // this lane's maximum over its 8 keys; some lane of a column exceeds the
       // column's running maximum by more than kLazy exactly when the column's
       // maximum does, so the lanes combine (two butterflies over the column's
       // four lane groups) only on the rare steps that rescale
-      float mx = fmaxf(fmaxf(fmaxf(sv[0], sv[1]), fmaxf(sv[2], sv[3])),
-                       fmaxf(fmaxf(sv[4], sv[5]), fmaxf(sv[6], sv[7])));
-      if (__ballot(mx * a.qk_scale_log2 > m_run[c] + kLazy)) {   // wave-uniform; the scale is positive
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = fmaxf(m_run[c], mx * a.qk_scale_log2);
+      mx[c] = fmaxf(fmaxf(fmaxf(sv[c][0], sv[c][1]), fmaxf(sv[c][2], sv[c][3])),
+                    fmaxf(fmaxf(sv[c][4], sv[c][5]), fmaxf(sv[c][6], sv[c][7])));
+      raise |= mx[c] * a.qk_scale_log2 > m_run[c] + kLazy;
+    }
+    if (__ballot(raise)) {   // wave-uniform; the scale is positive
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        if (!__ballot(mx[c] * a.qk_scale_log2 > m_run[c] + kLazy)) continue;
+        float m = fmaxf(mx[c], __shfl_xor(mx[c], 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        const float m_new = fmaxf(m_run[c], m * a.qk_scale_log2);
         const float alpha = __builtin_amdgcn_exp2f(m_run[c] - (m_new == -INFINITY ? 0.f : m_new));
         l_run[c] *= alpha;
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[c][d] *= alpha;
         m_run[c] = m_new;
       }
+    }
+    // P enters the PV product rounded to fp16, as the fp16 SDPA of the
+    // reference's prefill keeps it (the row sums stay fp32)
+    h8_t ph[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
       const float nref = m_run[c] == -INFINITY ? 0.f : -m_run[c];
-      // P enters the PV product rounded to fp16, as the fp16 SDPA of the
-      // reference's prefill keeps it (the row sums stay fp32)
-      h8_t ph;
       float lsum = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[j], a.qk_scale_log2, nref));
-        ph[j] = (_Float16)p;
+        const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(sv[c][j], a.qk_scale_log2, nref));
+        ph[c][j] = (_Float16)p;
         lsum += p;
       }
       l_run[c] += lsum;
+    }
 #pragma unroll
-      for (int d = 0; d < DT; ++d)
-        o[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf.v[d], ph, o[c][d], 0, 0, 0);
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        o[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(bf.v[d], ph[c], o[c][d], 0, 0, 0);
+  };
+  // SPLIT: this workgroup's share [lo, hi) of its rows' key steps
+  const int lo = SPLIT ? wg_steps * sp / a.S : 0;
+  const int hi = SPLIT ? wg_steps * (sp + 1) / a.S : wg_steps;
+  if (lo < hi) {
+    slots(lo);
+    issue(lo, 0);
+    slots(lo + 1);
+  }
+  // Every wave passes one barrier per step of the workgroup, whichever of the
+  // three loops it is in: steps without masking, steps with, and copies for the
+  // workgroup's later waves only.  (One loop with both forms in it spills.)
+  auto stage = [&](int s) {
+    stage_barrier();                 // tile s is in its stage; the other stage is no longer read
+    if (s + 1 < hi) {
+      issue(s + 1, (s + 1 - lo) & 1);
+      slots(s + 2);
     }
   };
-  auto step = [&](KStep<D>& bf, int s) {
-    if (s < nfull) compute(std::true_type{}, bf, s);
-    else compute(std::false_type{}, bf, s);
-  };
-
-  issue(0, 0);
-  for (int s = 0; s < wg_steps; ++s) {
-    stage_barrier();                 // tile s is in stage s&1; stage (s+1)&1 is no longer read
+  int s = lo;
+  for (; s < min(hi, nfull); ++s) {
+    stage(s);
     KStep<D> bf;
-    if (s < nsteps) read(bf, s, s & 1);
-    if (s + 1 < wg_steps) issue(s + 1, (s + 1) & 1);
-    if (s < nsteps) step(bf, s);
+    read(bf, (s - lo) & 1);
+    compute(std::true_type{}, bf, s);
   }
+  for (; s < min(hi, nsteps); ++s) {
+    stage(s);
+    KStep<D> bf;
+    read(bf, (s - lo) & 1);
+    compute(std::false_type{}, bf, s);
+  }
+  for (; s < hi; ++s) stage(s);
 
-  // normalise and store: o[c][d][r] = O^T[dim d*16 + grp*4 + r][query col of tile c]
+  // normalise and store: o[c][d][r] = O^T[dim d*16 + grp*4 + r][row col of tile c]
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     float l = l_run[c];
     l += __shfl_xor(l, 16, 64);
     l += __shfl_xor(l, 32, 64);
-    const int qi = qw + c * 16 + col;
-    if (qi < a.T) {
+    if (qw + c * 16 + col >= R) continue;
+    if constexpr (SPLIT) {
+      const int64_t pi = ((int64_t)tq[c] * a.Hq + hq[c]) * a.S + sp;
+      float* dst = a.part_o + pi * D + grp * 4;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) *reinterpret_cast<f4_t*>(dst + d * 16) = o[c][d];
+      if (grp == 0) *reinterpret_cast<float2*>(a.part_ml + pi * 2) = make_float2(m_run[c], l);
+    } else {
       const float inv = l > 0.f ? 1.f / fmaxf(l, 1e-12f) : 0.f;
-      uint16_t* dst = a.out + (int64_t)qi * a.o_st + (int64_t)h * a.o_sh + grp * 4;
+      uint16_t* dst = a.out + (int64_t)tq[c] * a.o_st + (int64_t)hq[c] * a.o_sh + grp * 4;
 #pragma unroll
       for (int d = 0; d < DT; ++d) {
-        const uint32_t lo = pack_h2(o[c][d][0] * inv, o[c][d][1] * inv);
-        const uint32_t hi = pack_h2(o[c][d][2] * inv, o[c][d][3] * inv);
-        *reinterpret_cast<uint2*>(dst + d * 16) = make_uint2(lo, hi);
+        const uint32_t w0 = pack_h2(o[c][d][0] * inv, o[c][d][1] * inv);
+        const uint32_t w1 = pack_h2(o[c][d][2] * inv, o[c][d][3] * inv);
+        *reinterpret_cast<uint2*>(dst + d * 16) = make_uint2(w0, w1);
       }
     }
   }
+}
+
+// Merges the key splits: out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s, four
+// dims per thread; bound by reading the partials once.
+template <int D>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
+  const int row = (int)(((int64_t)blockIdx.x * 256 + threadIdx.x) / (D / 4));
+  const int d = ((int)threadIdx.x % (D / 4)) * 4;
+  if (row >= a.T * a.Hq) return;
+  const float* ml = a.part_ml + (int64_t)row * a.S * 2;
+  const float* po = a.part_o + (int64_t)row * a.S * D + d;
+  float m = -INFINITY;
+  for (int s = 0; s < a.S; ++s) m = fmaxf(m, ml[2 * s]);
+  const float ref = m == -INFINITY ? 0.f : m;
+  float num[4] = {0.f, 0.f, 0.f, 0.f}, den = 0.f;
+  for (int s = 0; s < a.S; ++s) {
+    const float w = __builtin_amdgcn_exp2f(ml[2 * s] - ref);
+    const f4_t o = *reinterpret_cast<const f4_t*>(po + (int64_t)s * D);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) num[e] = fmaf(w, o[e], num[e]);
+    den = fmaf(w, ml[2 * s + 1], den);
+  }
+  const float inv = den > 0.f ? 1.f / fmaxf(den, 1e-12f) : 0.f;
+  const int t = row / a.Hq;
+  uint16_t* dst = a.out + (int64_t)t * a.o_st + (int64_t)(row - t * a.Hq) * a.o_sh + d;
+  *reinterpret_cast<uint2*>(dst) =
+      make_uint2(pack_h2(num[0] * inv, num[1] * inv), pack_h2(num[2] * inv, num[3] * inv));
+}
+
+// Key splits of a causal call.  A workgroup's steps are a serial chain of about a
+// microsecond each, so a grid that leaves workgroup slots empty is cut along the
+// keys, priced in steps: rounds of workgroups (two per CU) x the steps of a split
+// and its start, plus the partials' traffic and the merge launch.  From 129
+// workgroups on, up to 2048 keys stay one pass: little to gain, and a row's bits
+// then do not depend on how its prompt was chunked.
+int prefill_splits(int T, int q_start, int Hq, int Hkv, int D) {
+  const int64_t keys = (int64_t)q_start + T;
+  const int64_t blocks = ((int64_t)T * (Hq / Hkv) + 64 * PF_NC - 1) / (64 * PF_NC) * Hkv;
+  if (blocks >= 512 || (blocks > 128 && keys <= 2048)) return 1;
+  const int steps = (int)((keys + kKS - 1) / kKS);
+  const double part = (double)T * Hq * D * 8.0 / 4e6;      // us (about a step) per split
+  int best = 1;
+  double cost = -1.0;
+  for (int s = 1; s <= 32 && s <= std::max(1, steps / 4); ++s) {
+    const int64_t n = blocks * s;
+    const double rounds = n <= 256 ? 0.9 : (double)((n + 511) / 512);
+    const double c = rounds * ((steps + s - 1) / s + 3) + (s > 1 ? 3.0 + part * s : 0.0);
+    if (cost < 0.0 || c < 0.95 * cost) { cost = c; best = s; }
+  }
+  return best;
 }
 
 }  // namespace
@@ -400,7 +527,7 @@ int prefill_launch(const char* fn, const void* q, int64_t q_stride_t, int64_t q_
                    const helm_kv_pool* pool, const int32_t* page_table, int q_start, int T, int Hq,
                    int Hkv, int D, int P, float scale, void* out, int64_t out_stride_t,
                    int64_t out_stride_h, const void* mask, int64_t mask_stride_h,
-                   int64_t mask_stride_t, int kv_len, const int32_t* key_end, void* stream) {
+                   int64_t mask_stride_t, int kv_len, const int32_t* key_end, void* ws, int64_t ws_bytes, void* stream) {
   const std::string f(fn);
   HELM_CHECK_ARG(q && pool && pool->k && pool->v && page_table && out, f + ": null pointer");
   HELM_CHECK_ARG(T >= 1 && q_start >= 0 && Hq >= 1 && Hkv >= 1, f + ": bad sizes");
@@ -445,23 +572,38 @@ int prefill_launch(const char* fn, const void* q, int64_t q_stride_t, int64_t q_
   a.inv_scale = 1.f / scale;
   a.key_end = key_end;
   hipStream_t s = static_cast<hipStream_t>(stream);
+  a.S = mask ? 1 : prefill_splits(T, q_start, Hq, Hkv, D);
+  const int64_t rows = (int64_t)T * Hq * a.S;
+  if (!ws || !helm::aligned16(ws) || ws_bytes < rows * (D + 2) * (int64_t)sizeof(float)) a.S = 1;
+  a.part_o = static_cast<float*>(ws);
+  a.part_ml = a.part_o ? a.part_o + rows * D : nullptr;
   auto go = [&](auto kern) {
     constexpr int qb = 64 * PF_NC;
-    hipLaunchKernelGGL(kern, dim3(((T + qb - 1) / qb) * Hq), dim3(256), 0, s, a);
+    const int nqb = (int)(((int64_t)T * (Hq / Hkv) + qb - 1) / qb);
+    hipLaunchKernelGGL(kern, dim3(nqb * Hkv * a.S), dim3(256), 0, s, a);
   };
-  auto by_page = [&](auto d_tag, auto m_tag) {
+  auto by_page = [&](auto d_tag, auto m_tag, auto s_tag) {
     constexpr int Dc = decltype(d_tag)::value;
     constexpr bool Mc = decltype(m_tag)::value;
-    if (P == 16) go(prefill_attn_kernel<Dc, 16, PF_NC, Mc>);
-    else if (P == 32) go(prefill_attn_kernel<Dc, 32, PF_NC, Mc>);
-    else go(prefill_attn_kernel<Dc, 64, PF_NC, Mc>);
+    constexpr bool Sc = decltype(s_tag)::value;
+    if (P == 16) go(prefill_attn_kernel<Dc, 16, PF_NC, Mc, Sc>);
+    else if (P == 32) go(prefill_attn_kernel<Dc, 32, PF_NC, Mc, Sc>);
+    else go(prefill_attn_kernel<Dc, 64, PF_NC, Mc, Sc>);
   };
-  auto by_mask = [&](auto d_tag) {
-    if (mask) by_page(d_tag, std::true_type{});
-    else by_page(d_tag, std::false_type{});
+  auto by_dim = [&](auto d_tag) {
+    constexpr int Dc = decltype(d_tag)::value;
+    if (mask) {
+      by_page(d_tag, std::true_type{}, std::false_type{});
+    } else if (a.S > 1) {
+      by_page(d_tag, std::false_type{}, std::true_type{});
+      const int64_t threads = (int64_t)T * Hq * (Dc / 4);
+      hipLaunchKernelGGL((prefill_merge_kernel<Dc>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, a);
+    } else {
+      by_page(d_tag, std::false_type{}, std::false_type{});
+    }
   };
-  if (D == 64) by_mask(std::integral_constant<int, 64>{});
-  else by_mask(std::integral_constant<int, 128>{});
+  if (D == 64) by_dim(std::integral_constant<int, 64>{});
+  else by_dim(std::integral_constant<int, 128>{});
   HELM_CHECK_LAUNCH(fn);
   return HELM_OK;
 }
@@ -475,7 +617,23 @@ extern "C" int helm_prefill_attn(const void* q, int64_t q_stride_t, int64_t q_st
                                  void* stream) {
   return prefill_launch("helm_prefill_attn", q, q_stride_t, q_stride_h, pool, page_table, q_start,
                         T, Hq, Hkv, D, P, scale, out, out_stride_t, out_stride_h, nullptr, 0, 0, 0,
-                        nullptr, stream);
+                        nullptr, nullptr, 0, stream);
+}
+
+extern "C" int64_t helm_prefill_attn_workspace_bytes(int T, int q_start, int Hq, int Hkv, int D) {
+  if (T < 1 || q_start < 0 || Hkv < 1 || Hq < Hkv || Hq % Hkv != 0 || D < 1) return 0;
+  const int S = prefill_splits(T, q_start, Hq, Hkv, D);
+  return S > 1 ? (int64_t)T * Hq * S * (D + 2) * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int helm_prefill_attn_ws(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                                    const helm_kv_pool* pool, const int32_t* page_table,
+                                    int q_start, int T, int Hq, int Hkv, int D, int P, float scale,
+                                    void* out, int64_t out_stride_t, int64_t out_stride_h,
+                                    void* workspace, int64_t workspace_bytes, void* stream) {
+  return prefill_launch("helm_prefill_attn_ws", q, q_stride_t, q_stride_h, pool, page_table, q_start,
+                        T, Hq, Hkv, D, P, scale, out, out_stride_t, out_stride_h, nullptr, 0, 0, 0,
+                        nullptr, workspace, workspace_bytes, stream);
 }
 
 extern "C" int helm_prefill_attn_mask(const void* q, int64_t q_stride_t, int64_t q_stride_h,
@@ -488,5 +646,5 @@ extern "C" int helm_prefill_attn_mask(const void* q, int64_t q_stride_t, int64_t
   HELM_CHECK_ARG(mask, "helm_prefill_attn_mask: null mask");
   return prefill_launch("helm_prefill_attn_mask", q, q_stride_t, q_stride_h, pool, page_table, 0,
                         T, Hq, Hkv, D, P, scale, out, out_stride_t, out_stride_h, mask,
-                        mask_stride_h, mask_stride_t, kv_len, key_end, stream);
+                        mask_stride_h, mask_stride_t, kv_len, key_end, nullptr, 0, stream);
 }

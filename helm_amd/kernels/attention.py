@@ -430,9 +430,12 @@ def prefill_attention(q: torch.Tensor, pool: PoolView, page_table: torch.Tensor,
     if out is None:
         out = torch.empty(T, Hq, D, dtype=torch.float16, device=q.device)
     if mask is None:
-        _native.call("helm_prefill_attn", q.data_ptr(), q.stride(0), q.stride(1), pool.c_ref(),
+        need = int(_native.lib().helm_prefill_attn_workspace_bytes(T, int(q_start), Hq,
+                                                                   pool.num_kv_heads, D))
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
+        _native.call("helm_prefill_attn_ws", q.data_ptr(), q.stride(0), q.stride(1), pool.c_ref(),
                      page_table.data_ptr(), int(q_start), T, Hq, pool.num_kv_heads, D, page_size,
-                     float(scale), out.data_ptr(), out.stride(0), out.stride(1),
+                     float(scale), out.data_ptr(), out.stride(0), out.stride(1), _native.ptr(ws), need,
                      _native.stream_ptr(q.device))
         return out
     _native.require_cuda(mask, what="prefill_attention")

@@ -236,6 +236,19 @@ int helm_prefill_attn(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                       int q_start, int T, int Hq, int Hkv, int D, int P, float scale,
                       void* out, int64_t out_stride_t, int64_t out_stride_h, void* stream);
 
+/* helm_prefill_attn with a caller-owned workspace of
+ * helm_prefill_attn_workspace_bytes (16-byte aligned; its contents on entry do not
+ * matter): calls whose rows leave workgroup slots empty (few queries over many
+ * cached keys) then also split the keys, keep fp32 partials there and merge them in
+ * a second kernel.  Same results up to the fp32 summation order; without the
+ * workspace (null, or too small) as helm_prefill_attn. */
+int64_t helm_prefill_attn_workspace_bytes(int T, int q_start, int Hq, int Hkv, int D);
+int helm_prefill_attn_ws(const void* q, int64_t q_stride_t, int64_t q_stride_h,
+                         const helm_kv_pool* pool, const int32_t* page_table,
+                         int q_start, int T, int Hq, int Hkv, int D, int P, float scale,
+                         void* out, int64_t out_stride_t, int64_t out_stride_h,
+                         void* workspace, int64_t workspace_bytes, void* stream);
+
 /* Prefill attention of one sequence under an arbitrary additive mask: the T
  * queries q [T, Hq, D] attend keys 0 .. kv_len-1 of the pages page_table[0 ..
  * ceil(kv_len/P)) with softmax(scale * q.k + mask[h, t, key]).  mask is fp16,

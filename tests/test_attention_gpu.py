@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 import torch
 
+from helm_amd import _native
 from helm_amd.kernels import attention as ka
 from oracle import attention as oa
 
@@ -359,6 +360,50 @@ def test_prefill_attention_matches_causal_reference(Hq, Hkv, D, P, T, q_start):
     assert np.abs(got - ref).max() <= ATOL
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,P,T,q_start", [(32, 8, 128, 16, 19, 1500), (16, 8, 64, 32, 129, 333),
+                                                  (40, 8, 128, 64, 5, 2100), (8, 1, 128, 16, 1, 4095),
+                                                  (64, 8, 64, 16, 33, 700), (10, 2, 128, 16, 26, 395)])
+def test_prefill_attention_key_splits(Hq, Hkv, D, P, T, q_start):
+    """Few queries over many cached keys: the keys are cut into splits merged by a
+    second kernel (helm_prefill_attn_ws), rows of a group packed into one block
+    (odd T, groups of 2, 4, 5 and 8, one row, a last split ending inside a step).
+    Against the fp64 causal form, and against the one-pass form without a
+    workspace; strided q and out; a workspace that starts as NaN."""
+    g = np.random.default_rng(T + q_start + D)
+    N = q_start + T
+    n_pages = (N + P - 1) // P
+    k_all = g.standard_normal((N, Hkv, D)).astype(np.float16)
+    v_all = g.standard_normal((N, Hkv, D)).astype(np.float16)
+    kp = np.full((n_pages + 3, Hkv, P, D), np.nan, np.float16)
+    vp = np.full((n_pages + 3, Hkv, P, D), np.nan, np.float16)
+    pt = g.permutation(n_pages + 3)[:n_pages].astype(np.int32)
+    for t in range(N):
+        kp[pt[t // P], :, t % P] = k_all[t]
+        vp[pt[t // P], :, t % P] = v_all[t]
+    q = g.standard_normal((T, Hq, D)).astype(np.float16)
+    scale = 1.0 / math.sqrt(D)
+    dev = torch.device("cuda")
+    pool = device_pool(kp, vp)
+    qd = torch.from_numpy(q).to(dev).transpose(0, 1).contiguous().transpose(0, 1)   # head-major storage
+    ptd = torch.from_numpy(pt).to(dev)
+    need = _native.lib().helm_prefill_attn_workspace_bytes(T, q_start, Hq, Hkv, D)
+    assert need > 0
+    ref = oa.causal_prefill_reference(q, k_all, v_all, q_start, scale)
+    outs = []
+    for bytes_ in (need, 0):
+        ws = torch.full((need // 4,), float("nan"), device=dev)
+        out = torch.full((T, Hq, D + 4), float("nan"), dtype=torch.float16, device=dev)
+        _native.call("helm_prefill_attn_ws", qd.data_ptr(), qd.stride(0), qd.stride(1), pool.c_ref(),
+                     ptd.data_ptr(), q_start, T, Hq, Hkv, D, P, scale, out.data_ptr(), out.stride(0),
+                     out.stride(1), ws.data_ptr(), bytes_, torch.cuda.current_stream().cuda_stream)
+        assert torch.isnan(out[..., D:]).all()
+        outs.append(out[..., :D].cpu().numpy().astype(np.float64))
+    outs.append(ka.prefill_attention(qd, pool, ptd, P, q_start, scale).cpu().numpy().astype(np.float64))
+    for o in outs:
+        assert np.abs(o - ref).max() <= ATOL
+    assert np.array_equal(outs[0], outs[2])
+
+
 def _mask_case(kind, Hq, T, N, g):
     """Masks of the shapes a drop-in prefill receives: [Hm, T, N]."""
     causal = np.arange(N)[None, :] <= np.arange(T)[:, None] + (N - T)
@@ -624,3 +669,42 @@ def test_qk_norm_rope_cs_matches_transformers_ops(norm, shared_rows, rope_scalin
         bound = 2.0 ** -10 * terms + 2.0 ** (np.floor(np.log2(mag)) - 10)
         assert (np.abs(g64 - r64) <= bound).all(), float(np.abs(g64 - r64).max())
         assert (g64 == r64).mean() > 0.99
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,P,first,scatter", [(64, 32, 8, 128, 16, 0, False), (200, 40, 8, 128, 16, 5, False),
+                                                        (133, 16, 8, 64, 32, 8, False), (99, 5, 1, 128, 64, 24, False),
+                                                        (150, 6, 3, 64, 16, 3, True), (65, 9, 9, 128, 8, 0, False)])
+def test_qk_norm_rope_append_prompt_form_equals_row_form(T, Hq, Hkv, D, P, first, scatter):
+    """helm_qk_norm_rope_append's prompt form (64 tokens on) writes the same bits as
+    its per-row form (the same tokens in calls of 48): a prompt from any offset of
+    its first page, tokens in scattered pages, rejected slots and offsets, head
+    counts that do not fill the eight of a workgroup."""
+    from helm_amd.kernels import fused
+    dev = torch.device("cuda")
+    g = torch.Generator(device=dev).manual_seed(T + D)
+    n_pages = (first + T + P - 1) // P
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, generator=g, device=dev).half()
+    qn, kn = ((1 + 0.1 * torch.randn(D, generator=g, device=dev)).half() for _ in range(2))
+    at = torch.arange(first, first + T, device=dev)
+    perm = torch.randperm(n_pages + 2, generator=g, device=dev).int()
+    if scatter:
+        at = at[torch.randperm(T, generator=g, device=dev)]
+    slots, offs = perm[at // P].contiguous(), (at % P).int()
+    slots[T // 2], offs[T // 3], slots[T - 1] = -1, P, n_pages + 2
+    pos = (at + 40000).int()
+    inv = fused.rope_inv_freq(D, 1e6, dev)
+    outs = []
+    for step in (T, 48):
+        k = torch.full((n_pages + 2, Hkv, P, D), 7.0, dtype=torch.float16, device=dev)
+        v = ka.alloc_v((n_pages + 2, Hkv, P, D), device=dev)
+        v.fill_(7.0)
+        q_out = torch.zeros(T, Hq, D, dtype=torch.float16, device=dev)
+        pool = ka.PoolView.of_pool(k, v)
+        for i in range(0, T, step):
+            j = slice(i, min(T, i + step))
+            fused.qk_norm_rope_append(qkv[j], qn, kn, 1e-6, pos[j], inv, q_out[j], pool, slots[j], offs[j],
+                                      Hq, Hkv, D, P)
+        outs.append((q_out, k, v))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    assert not torch.equal(outs[0][1], torch.full_like(outs[0][1], 7.0))
