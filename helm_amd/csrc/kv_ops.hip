@@ -138,6 +138,224 @@ __global__ __launch_bounds__(256) void qk_norm_rope_append_kernel(
   }
 }
 
+// The same for a prompt's tokens.  Bound by moving qkv once through HBM; the form
+// above spends most of its time elsewhere: a 2-byte store per V element, each in
+// its own cache line, and a sine and a cosine per element of every head.  Here a
+// workgroup takes 16 tokens x 8 heads:
+//   * q / k heads: the RoPE factors of the 16 tokens are computed once into LDS; a
+//     lane holds 8 dims of a row (16-byte loads and stores, D / 8 lanes a row), all
+//     rows of a wave requested before the first is used.  The sum of squares adds
+//     in the order of wave_sum over lanes l = d mod 64, so rows equal the per-row
+//     form's (and the fused decode attention's) bit for bit;
+//   * v heads: 16 tokens of a head are transposed through LDS; where they fill
+//     aligned runs of one page (a prompt written from a multiple of 8 on), each dim's
+//     8 tokens go out as one 16-byte store, elsewhere token by token.
+// 2000 tokens, 32 + 16 heads of 128: 39.5 -> 15.1 us (3.3 TB/s of the 49 MB); 4096
+// tokens, 64 + 16 heads: 123 -> 35.7 us (4.7 TB/s).
+constexpr int kTT = 16;       // tokens of a workgroup
+constexpr int kHC = 8;        // heads of a workgroup
+// fewest tokens: a workgroup's chain (factors, then four rounds of rows) takes about 6
+// us however few there are; the per-row form 4.9 us at 128 tokens (here 6.3), 9.4
+// at 300 (here 6.8)
+constexpr int kPromptMin = 192;
+
+constexpr int kPW = 8;        // waves of a workgroup
+
+// v of the lane that DPP control CTRL names
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __builtin_bit_cast(float, dpp_u<CTRL>(__builtin_bit_cast(uint32_t, v)));
+}
+
+template <int D>
+__global__ __launch_bounds__(kPW * 64) void qk_norm_rope_append_prompt_kernel(
+    const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ q_norm_w,
+    const uint16_t* __restrict__ k_norm_w, float eps, const int32_t* __restrict__ positions,
+    const float* __restrict__ inv_freq, uint16_t* __restrict__ q_out, PoolArgs pa,
+    const int32_t* __restrict__ slots, const int32_t* __restrict__ offsets, int B, int Hq, int Hkv,
+    int P, bool v_vec) {
+  constexpr int HALF = D / 2;
+  constexpr int LPR = D / 8;                   // lanes of a row
+  constexpr int RPW = 64 / LPR;                // rows of a wave at a time
+  constexpr int IT = kTT * kHC / (kPW * RPW);    // row rounds of a wave
+  constexpr int kVP = D / 2 + 1;               // V staging pitch (dwords)
+  __shared__ uint32_t s_cs[kTT][HALF];         // cos | sin << 16, fp16 bits
+  __shared__ int s_slot[kTT], s_off[kTT];
+  __shared__ uint32_t s_v[kPW][kTT * kVP];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  const int b0 = blockIdx.x * kTT;
+  const int nt = min(kTT, B - b0);
+  const int heads = Hq + 2 * Hkv;
+  const int qk_chunks = (Hq + Hkv + kHC - 1) / kHC;
+  if (tid < kTT) {
+    const int b = min(b0 + tid, B - 1);
+    const int slot = slots[b], off = offsets[b];
+    const bool ok = slot >= 0 && slot < pa.num_slots && off >= 0 && off < P;
+    s_slot[tid] = ok ? slot : -1;
+    s_off[tid] = off;
+  }
+
+  if ((int)blockIdx.y >= qk_chunks) {          // value heads (uniform over the workgroup)
+    __syncthreads();
+    const int h0 = ((int)blockIdx.y - qk_chunks) * kHC;
+    uint32_t* sv = s_v[wave];
+    // 8-token runs that are one aligned run of a valid page
+    bool run[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      run[g] = v_vec && 8 * g + 8 <= nt && s_slot[8 * g] >= 0 && s_off[8 * g] % 8 == 0 && s_off[8 * g] + 8 <= P;
+#pragma unroll
+      for (int t = 1; t < 8; ++t)
+        run[g] = run[g] && s_slot[8 * g + t] == s_slot[8 * g] && s_off[8 * g + t] == s_off[8 * g] + t;
+    }
+    for (int h = h0 + wave; h < min(h0 + kHC, Hkv); h += kPW) {
+#pragma unroll
+      for (int i = 0; i < kTT * LPR / 64; ++i) {
+        const int c = i * 64 + lane;
+        const int t = c / LPR, d8 = c % LPR;
+        const uint4 v = *reinterpret_cast<const uint4*>(
+            qkv + ((int64_t)min(b0 + t, B - 1) * heads + Hq + Hkv + h) * D + d8 * 8);
+        uint32_t* dst = sv + t * kVP + d8 * 4;
+        dst[0] = v.x; dst[1] = v.y; dst[2] = v.z; dst[3] = v.w;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      if (lane < HALF) {                       // dims 2 lane, 2 lane + 1 (D = 128: all lanes)
+        uint32_t w[kTT];
+#pragma unroll
+        for (int t = 0; t < kTT; ++t) w[t] = sv[t * kVP + lane];
+        uint16_t* vh = pa.v + (int64_t)h * pa.v_hs + (int64_t)(2 * lane) * pa.v_ds;
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          if (run[g]) {
+            uint16_t* dst = vh + (int64_t)s_slot[8 * g] * pa.v_ss + s_off[8 * g];
+            uint32_t lo[4], hi[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const uint32_t p0 = w[8 * g + 2 * j], p1 = w[8 * g + 2 * j + 1];
+              lo[j] = (p0 & 0xffffu) | (p1 << 16);
+              hi[j] = (p0 >> 16) | (p1 & 0xffff0000u);
+            }
+            *reinterpret_cast<uint4*>(dst) = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+            *reinterpret_cast<uint4*>(dst + pa.v_ds) = make_uint4(hi[0], hi[1], hi[2], hi[3]);
+          } else {
+#pragma unroll
+            for (int t = 8 * g; t < 8 * g + 8; ++t) {
+              if (t >= nt || s_slot[t] < 0) continue;
+              uint16_t* dst = vh + (int64_t)s_slot[t] * pa.v_ss + s_off[t];
+              dst[0] = (uint16_t)(w[t] & 0xffffu);
+              dst[pa.v_ds] = (uint16_t)(w[t] >> 16);
+            }
+          }
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      __builtin_amdgcn_wave_barrier();         // the staging is rewritten by this wave's next head
+    }
+    return;
+  }
+
+  // query and key heads: row r of the workgroup is token r / kHC, head h0 + r % kHC
+  const int h0 = (int)blockIdx.y * kHC;
+  const int nh = min(kHC, Hq + Hkv - h0);
+  // this lane's dims 8 li .. + 8 of its row: bits 0 and 2 of the lane swapped, so
+  // that each exchange below is one DPP control
+  const int li = (lane & (LPR - 1) & ~5) | ((lane & 1) << 2) | ((lane >> 2) & 1);
+  uint4 xr[IT];
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int r = (i * kPW + wave) * RPW + lane / LPR;
+    const int t = r / kHC, h = h0 + min(r % kHC, nh - 1);
+    xr[i] = *reinterpret_cast<const uint4*>(qkv + ((int64_t)min(b0 + t, B - 1) * heads + h) * D + li * 8);
+  }
+  for (int i = tid; i < kTT * HALF; i += kPW * 64) {
+    const int t = i / HALF, d = i % HALF;
+    const float ang = inv_freq[d] * (float)positions[min(b0 + t, B - 1)];
+    s_cs[t][d] = (uint32_t)f2h(cosf(ang)) | ((uint32_t)f2h(sinf(ang)) << 16);
+  }
+  const uint4 qw = *reinterpret_cast<const uint4*>(q_norm_w + li * 8);
+  const uint4 kw = *reinterpret_cast<const uint4*>(k_norm_w + li * 8);
+  __syncthreads();
+  constexpr int PX = LPR / 2;                  // lane holding dims d +- D/2
+  const bool low = li < PX;
+#pragma unroll
+  for (int i = 0; i < IT; ++i) {
+    const int r = (i * kPW + wave) * RPW + lane / LPR;
+    const int t = r / kHC, hi_ = r % kHC, h = h0 + min(hi_, nh - 1);
+    const uint32_t wd[4] = {xr[i].x, xr[i].y, xr[i].z, xr[i].w};
+    float x[8], v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = h2f((uint16_t)(wd[e >> 1] >> (16 * (e & 1))));
+    // squares in wave_sum's order: lane l = d mod 64, then offsets 32 .. 1
+    if constexpr (D == 128) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t o = dpp_u<0x128>(wd[j]);      // row_ror:8 = dims +- 64
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float mine = x[2 * j + e], other = h2f((uint16_t)(o >> (16 * e)));
+          const float a = low ? mine : other, b = low ? other : mine;
+          v[2 * j + e] = fmaf(b, b, a * a);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = x[e] * x[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      v[e] = dpp_add<0xB1>(v[e]);     // l ^ 32: quad_perm [1,0,3,2]
+      v[e] = dpp_add<0x4E>(v[e]);     // l ^ 16: quad_perm [2,3,0,1]
+      v[e] = dpp_add<0x141>(v[e]);    // l ^ 8: row_half_mirror (the quad's lanes agree)
+    }
+    float v4[4], v2[2];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v4[e] = v[e] + v[e + 4];
+    v2[0] = v4[0] + v4[2];
+    v2[1] = v4[1] + v4[3];
+    const float rstd = rsqrtf((v2[0] + v2[1]) / (float)D + eps);
+    const bool is_q = h < Hq;
+    const uint4 nw = is_q ? qw : kw;
+    const uint32_t nwd[4] = {nw.x, nw.y, nw.z, nw.w};
+    uint32_t xn[4], out[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float t0 = h2f(f2h(x[2 * j] * rstd)), t1 = h2f(f2h(x[2 * j + 1] * rstd));
+      xn[j] = pack_h2(lo_h(nwd[j]) * t0, hi_h(nwd[j]) * t1);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t o = D == 128 ? dpp_u<0x128>(xn[j]) : dpp_u<0xB1>(xn[j]);
+      float res[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+#pragma clang fp contract(off)   // each product is rounded to fp16 before the sum
+        const uint32_t cs = s_cs[t][(li * 8 + 2 * j + e) % HALF];
+        const float mine = e ? hi_h(xn[j]) : lo_h(xn[j]);
+        const float partner = e ? hi_h(o) : lo_h(o);
+        const float rot = low ? -partner : partner;
+        const float t1 = h2f(f2h(mine * lo_h(cs)));
+        const float t2 = h2f(f2h(rot * hi_h(cs)));
+        res[e] = t1 + t2;
+      }
+      out[j] = pack_h2(res[0], res[1]);
+    }
+    if (t >= nt || hi_ >= nh) continue;
+    const uint4 ov = make_uint4(out[0], out[1], out[2], out[3]);
+    if (is_q) {
+      *reinterpret_cast<uint4*>(q_out + ((int64_t)(b0 + t) * Hq + h) * D + li * 8) = ov;
+    } else if (s_slot[t] >= 0) {
+      *reinterpret_cast<uint4*>(pa.k + (int64_t)s_slot[t] * pa.k_ss + (int64_t)(h - Hq) * pa.k_hs +
+                                (int64_t)s_off[t] * D + li * 8) = ov;
+    }
+  }
+}
+
 // helm_qk_norm_rope_cs: one wave per (item, q or k head) of the fused qkv
 // output: the per-head RMSNorm when norm weights are given, then RoPE with the
 // caller's cos / sin rows (transformers' position embeddings, so every RoPE
@@ -599,6 +817,22 @@ extern "C" int helm_qk_norm_rope_append(const void* qkv, const void* q_norm_w, c
   const int blocks = (items + 3) / 4;
   const PoolArgs pa = pool_args(pool);
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // the prompt form from kPromptMin tokens on, where 16-byte accesses are aligned
+  if (B >= kPromptMin && helm::aligned16(qkv) && helm::aligned16(q_out) && helm::aligned16(q_norm_w) &&
+      helm::aligned16(k_norm_w)) {
+    const bool v_vec = helm::aligned16(pa.v) && pa.v_ss % 8 == 0 && pa.v_hs % 8 == 0 && pa.v_ds % 8 == 0;
+    const dim3 grid((B + kTT - 1) / kTT, (Hq + Hkv + kHC - 1) / kHC + (Hkv + kHC - 1) / kHC);
+    auto prompt = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(kPW * 64), 0, s, static_cast<const uint16_t*>(qkv),
+                         static_cast<const uint16_t*>(q_norm_w), static_cast<const uint16_t*>(k_norm_w),
+                         eps, positions, inv_freq, static_cast<uint16_t*>(q_out), pa, slots, offsets, B,
+                         Hq, Hkv, P, v_vec);
+    };
+    if (D == 64) prompt(qk_norm_rope_append_prompt_kernel<64>);
+    else prompt(qk_norm_rope_append_prompt_kernel<128>);
+    HELM_CHECK_LAUNCH("helm_qk_norm_rope_append launch");
+    return HELM_OK;
+  }
   auto args = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, static_cast<const uint16_t*>(qkv),
                        static_cast<const uint16_t*>(q_norm_w), static_cast<const uint16_t*>(k_norm_w),

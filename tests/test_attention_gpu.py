@@ -671,11 +671,11 @@ def test_qk_norm_rope_cs_matches_transformers_ops(norm, shared_rows, rope_scalin
         assert (g64 == r64).mean() > 0.99
 
 
-@pytest.mark.parametrize("T,Hq,Hkv,D,P,first,scatter", [(64, 32, 8, 128, 16, 0, False), (200, 40, 8, 128, 16, 5, False),
-                                                        (133, 16, 8, 64, 32, 8, False), (99, 5, 1, 128, 64, 24, False),
-                                                        (150, 6, 3, 64, 16, 3, True), (65, 9, 9, 128, 8, 0, False)])
+@pytest.mark.parametrize("T,Hq,Hkv,D,P,first,scatter", [(192, 32, 8, 128, 16, 0, False), (200, 40, 8, 128, 16, 5, False),
+                                                        (233, 16, 8, 64, 32, 8, False), (199, 5, 1, 128, 64, 24, False),
+                                                        (250, 6, 3, 64, 16, 3, True), (305, 9, 9, 128, 8, 0, False)])
 def test_qk_norm_rope_append_prompt_form_equals_row_form(T, Hq, Hkv, D, P, first, scatter):
-    """helm_qk_norm_rope_append's prompt form (64 tokens on) writes the same bits as
+    """helm_qk_norm_rope_append's prompt form (192 tokens on) writes the same bits as
     its per-row form (the same tokens in calls of 48): a prompt from any offset of
     its first page, tokens in scattered pages, rejected slots and offsets, head
     counts that do not fill the eight of a workgroup."""
@@ -708,3 +708,4 @@ def test_qk_norm_rope_append_prompt_form_equals_row_form(T, Hq, Hkv, D, P, first
     for a, b in zip(*outs):
         assert torch.equal(a, b)
     assert not torch.equal(outs[0][1], torch.full_like(outs[0][1], 7.0))
+
