@@ -32,6 +32,7 @@ _SIGNATURES = {
     "helm_int8_gemv_swiglu": [_vp, _i64, _vp, _f32, _vp, _vp, _vp, _vp, _i64, _vp, _i64,
                               _i32, _i32, _i32, _vp],
     "helm_int8_gemm": [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp],
+    "helm_int8_gemm_ws": [_vp, _i64, _vp, _i64, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i64, _vp],
     "helm_paged_decode_attn": [_vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _i32, _i32,
                                _i32, _i32, _i32, _i32, _i32, _i32, _i32, _f32, _vp],
     "helm_decode_attn_fused": [_vp, _i64, _vp, _vp, _f32, _vp, _vp, _vp, _vp, _vp, _vp, _i64,
@@ -71,6 +72,7 @@ _OTHER = {
     "helm_argmax_workspace_bytes": ([_i32], _i64),
     "helm_prefill_attn_workspace_bytes": ([_i32, _i32, _i32, _i32, _i32], _i64),
     "helm_int8_gemv_workspace_bytes": ([_i32, _i32, _i32], _i64),
+    "helm_int8_gemm_workspace_bytes": ([_i32, _i32, _i32], _i64),
     "helm_int8_gemv_split_bytes": ([_i32, _i32, _i32], _i64),
 }
 

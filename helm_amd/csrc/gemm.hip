@@ -15,6 +15,7 @@
 // K-step.  LDS rows are XOR-swizzled in 16-byte chunks so that the operand reads
 // (16 rows at one k offset per instruction) hit every bank once.  The per-channel
 // scale and bias are applied once in the epilogue.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -26,11 +27,9 @@ typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
-constexpr int BM = 128, BK = 64;
+constexpr int BM = 128, BK = 64;            // BM: rows of the prompt form's tile
 constexpr int kThreads = 256;
-constexpr int kStages = 3;
-constexpr int kABytes = BM * BK * 2;        // fp16 x tile of one stage (16 KiB)
-constexpr int kAWaveCopies = kABytes / 1024 / 4;   // 1 KiB copies per wave (4)
+constexpr int kStages = 3;                  // ring stages of the prompt form
 
 // LDS swizzles (16-byte chunks): an operand read takes one chunk of 16 consecutive
 // rows (one 256-byte pass of the 64 4-byte banks); these make the 16 chunks
@@ -38,8 +37,11 @@ constexpr int kAWaveCopies = kABytes / 1024 / 4;   // 1 KiB copies per wave (4)
 __device__ __forceinline__ int aswz(int r) { return (r >> 1) & 7; }   // 128-byte rows
 __device__ __forceinline__ int bswz(int n) { return (n >> 2) & 3; }   // 64-byte rows
 
-template <int TN>
+// RT: row tiles of a wave without the k split; the workgroup's tile has 32 RT rows
+template <int TN, int RT>
 struct GemmCfg {
+  static constexpr int kABytes = 32 * RT * BK * 2;       // fp16 x tile of one stage
+  static constexpr int kAWaveCopies = kABytes / 1024 / 4;   // 1 KiB copies per wave
   static constexpr int BN = 32 * TN;
   static constexpr int kBBytes = BN * BK;                // int8 weight tile of one stage
   static constexpr int kStageBytes = kABytes + kBBytes;
@@ -79,13 +81,18 @@ __device__ __forceinline__ void lds_read_barrier() {
 // wave / 2) instead of the rows, so every int8 B fragment is dequantised once;
 // each wave then holds the partial sums of all 128 rows, and the pair adds them
 // through LDS after the last step.
-template <int TN, bool KSPLIT>
-__global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
+//
+// NS: ring stages (NS - 1 K-steps in flight).  PART: blockIdx.z takes K-steps
+// [z nk / S, (z + 1) nk / S) and writes fp32 partial sums to part [S, M, N].
+template <int TN, bool KSPLIT, int RT = 4, int NS = kStages, bool PART = false, int OCC = 2>
+__global__ __launch_bounds__(kThreads, OCC) void int8_gemm_kernel(
     const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ q, int64_t ldq,
     const uint16_t* __restrict__ scale, const uint16_t* __restrict__ bias, uint16_t* __restrict__ y,
-    int64_t ldy, int M, int N, int K) {
-  using C = GemmCfg<TN>;
-  constexpr int kRing = kStages * C::kStageBytes;
+    int64_t ldy, int M, int N, int K, float* __restrict__ part) {
+  using C = GemmCfg<TN, RT>;
+  static_assert(!KSPLIT || (RT == 4 && !PART), "the k split is built for 128-row tiles");
+  constexpr int kABytes = C::kABytes, kAWaveCopies = C::kAWaveCopies;
+  constexpr int kRing = NS * C::kStageBytes;
   constexpr int kRed = KSPLIT ? 4 * 4 * TN * 64 * 16 : 0;   // partial tiles handed to the partner
   __shared__ __attribute__((aligned(1024))) uint8_t smem[kRing > kRed ? kRing : kRed];
 
@@ -94,13 +101,14 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
   const int lane = tid & 63;
   const int col = lane & 15;
   const int grp = lane >> 4;
-  const int m0 = blockIdx.y * BM;
+  const int m0 = blockIdx.y * (32 * RT);
   const int n0 = blockIdx.x * C::BN;
-  constexpr int RI = KSPLIT ? 8 : 4;     // 16-row tiles of one wave
+  constexpr int RI = KSPLIT ? 8 : RT;    // 16-row tiles of one wave
   const int kh = wave >> 1;              // KSPLIT: k half of every K-step
-  const int wm = KSPLIT ? 0 : (wave >> 1) * 64;
+  const int wm = KSPLIT ? 0 : (wave >> 1) * (16 * RT);
   const int wn = (wave & 1) * (16 * TN);
-  const int nk = K / BK;
+  const int kb0 = PART ? (int)((int64_t)(K / BK) * blockIdx.z / gridDim.z) : 0;
+  const int nk = (PART ? (int)((int64_t)(K / BK) * (blockIdx.z + 1) / gridDim.z) : K / BK) - kb0;
 
   // Copy sources.  A stage: row r (128 B) holds logical chunk g (8 halves) in slot
   // g ^ aswz(r).  B stage: row n (64 B) holds logical chunk g (16 int8) in slot
@@ -113,7 +121,7 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
     const int c = (wave * kAWaveCopies + i) * 64 + lane;
     const int r = c >> 3;
     const int g = (c & 7) ^ aswz(r);
-    asrc[i] = x + (int64_t)min(m0 + r, M - 1) * ldx + g * 8;
+    asrc[i] = x + (int64_t)min(m0 + r, M - 1) * ldx + g * 8 + (int64_t)kb0 * BK;
   }
   const int8_t* bsrc[C::kBWaveMax];
 #pragma unroll
@@ -122,7 +130,7 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
     const int c = j * 64 + lane;
     const int n = c >> 2;
     const int g = (c & 3) ^ bswz(n);
-    bsrc[i] = q + (int64_t)min(n0 + n, N - 1) * ldq + g * 16;
+    bsrc[i] = q + (int64_t)min(n0 + n, N - 1) * ldq + g * 16 + (int64_t)kb0 * BK;
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_void_t*)smem;
   auto copy = [&](int kb, int st) {
@@ -192,11 +200,11 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
       const int n = wn + 16 * j + col;
       braw[j] = *reinterpret_cast<const uint4*>(Bs + n * 64 + ((grp ^ bswz(n)) << 4));
     }
-    h8_t af[2][4];
+    h8_t af[2][RI];
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+      for (int i = 0; i < RI; ++i) {
         const int r = wm + 16 * i + col;
         af[h][i] = *reinterpret_cast<const h8_t*>(As + r * 128 + (((2 * grp + h) ^ aswz(r)) << 4));
       }
@@ -214,25 +222,30 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < RI; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
           acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[h][i], bf[j][h], acc[i][j], 0, 0, 0);
   };
 
-  // Three-stage ring: copies of steps kb + 1 and kb + 2 are in flight while kb is
+  // Ring of NS stages: copies of steps kb + 1 .. kb + NS - 1 are in flight while kb is
   // consumed.  Before the barrier of step kb each wave waits until only its copies
-  // of step kb + 1 may still be outstanding (vector memory operations retire in
-  // order); after it, stage (kb + 2) % 3, last read in step kb - 1, is refilled.
-  copy(0, 0);
-  if (nk > 1) copy(1, 1);
+  // of the NS - 2 later steps may still be outstanding (vector memory operations
+  // retire in order; the last steps wait for all); after it, the stage last read in
+  // step kb - 1 is refilled with step kb + NS - 1.
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i)
+    if (i < nk) copy(i, i);
+  int st = 0, fill = NS - 1;
   for (int kb = 0; kb < nk; ++kb) {
-    if (kb + 1 < nk) wait_vm<C::kCopiesMin>();
+    if (kb + NS - 2 < nk) wait_vm<(NS - 2) * C::kCopiesMin>();
     else wait_vm<0>();
     lds_read_barrier();
-    if (kb + 2 < nk) copy(kb + 2, (kb + 2) % kStages);
-    if constexpr (KSPLIT) compute_ks(kb % kStages);
-    else compute(kb % kStages);
+    if (kb + NS - 1 < nk) copy(kb + NS - 1, fill);
+    if constexpr (KSPLIT) compute_ks(st);
+    else compute(st);
+    st = st + 1 == NS ? 0 : st + 1;
+    fill = fill + 1 == NS ? 0 : fill + 1;
   }
 
   if constexpr (KSPLIT) {
@@ -277,23 +290,52 @@ __global__ __launch_bounds__(kThreads, 2) void int8_gemm_kernel(
   for (int j = 0; j < TN; ++j) {
     const int n = n0 + wn + j * 16 + col;
     if (n >= N) continue;
-    const float sc = h2f(scale[n]);
-    const float bs = bias ? h2f(bias[n]) : 0.f;
+    const float sc = PART ? 0.f : h2f(scale[n]);
+    const float bs = !PART && bias ? h2f(bias[n]) : 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < RI; ++i) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wm + i * 16 + grp * 4 + r;
-        if (m < M) y[(int64_t)m * ldy + n] = f2h(acc[i][j][r] * sc + bs);
+        if (m >= M) continue;
+        if constexpr (PART) part[((int64_t)blockIdx.z * M + m) * N + n] = acc[i][j][r];
+        else y[(int64_t)m * ldy + n] = f2h(acc[i][j][r] * sc + bs);
       }
     }
   }
 }
 
+// Second pass of the split form: adds the S partial sums of an output, scale, bias,
+// one rounding to fp16; V consecutive outputs of a row per thread (N % V == 0).
+template <int V>
+__global__ __launch_bounds__(256) void gemm_split_reduce_kernel(
+    const float* __restrict__ part, int S, const uint16_t* __restrict__ scale,
+    const uint16_t* __restrict__ bias, uint16_t* __restrict__ y, int64_t ldy, int M, int N) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
+  if (i >= (int64_t)M * N) return;
+  const int m = (int)(i / N), n = (int)(i - (int64_t)m * N);
+  float v[V];
+#pragma unroll
+  for (int e = 0; e < V; ++e) v[e] = 0.f;
+  for (int s = 0; s < S; ++s) {
+    const float* p = part + (int64_t)s * M * N + i;
+    if constexpr (V == 4) {
+      const f4_t o = *reinterpret_cast<const f4_t*>(p);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] += o[e];
+    } else {
+      v[0] += p[0];
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < V; ++e)
+    y[(int64_t)m * ldy + n + e] = f2h(v[e] * h2f(scale[n + e]) + (bias ? h2f(bias[n + e]) : 0.f));
+}
+
 template <int TN>
 void launch_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq, const void* scale,
                  const void* bias, void* y, int64_t ldy, int M, int N, int K, hipStream_t s) {
-  dim3 grid((N + GemmCfg<TN>::BN - 1) / GemmCfg<TN>::BN, (M + BM - 1) / BM);
+  dim3 grid((N + 32 * TN - 1) / (32 * TN), (M + BM - 1) / BM);
   // K split from TN = 4 on (14B shapes, same-run A/B: 5120->5120 127.4 -> 120.3 us,
   // 17408->5120 364.2 -> 336.5 us); with TN = 2 the grid holds one workgroup per
   // CU and the split measured 3% slower.  HELM_GEMM_KSPLIT=0 turns it off.
@@ -301,11 +343,11 @@ void launch_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq, const
   if (ks_env && TN >= 4)
     hipLaunchKernelGGL((int8_gemm_kernel<TN, true>), grid, dim3(kThreads), 0, s,
                        static_cast<const uint16_t*>(x), ldx, q, ldq, static_cast<const uint16_t*>(scale),
-                       static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K);
+                       static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, nullptr);
   else
     hipLaunchKernelGGL((int8_gemm_kernel<TN, false>), grid, dim3(kThreads), 0, s,
                        static_cast<const uint16_t*>(x), ldx, q, ldq, static_cast<const uint16_t*>(scale),
-                       static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K);
+                       static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, nullptr);
 }
 
 int env_tn() {
@@ -335,23 +377,126 @@ int pick_tn(int M, int N) {
   return best;
 }
 
-}  // namespace
+// ---- few rows -------------------------------------------------------------
+// From 17 tokens up to a few tiles of rows a K-step is a chain of latencies (barrier,
+// LDS reads, dequantisation, MFMAs: 0.35-0.5 us whatever the copies in flight; a
+// ring of 7-12 stages at one workgroup per CU gave 31 of the 33 us at 77 x 4096 ->
+// 12288), so what counts is how many chains run at once and how long each is.  Here
+// tiles are 64 columns wide and as tall as the rows need (32 RT), two to four
+// workgroups fit a CU, and K is split over workgroups until they fill, partial sums
+// in fp32.  Against the prompt form alone, us: 77 tokens 17408 -> 5120 126 -> 43, 4096
+// -> 4096 32.4 -> 16.8, 4096 -> 1024 32.2 -> 12.0, 4096 -> 12288 33.5 -> 29.9; 17 tokens
+// 4096 -> 12288 33.4 -> 19.9; 256 tokens 17408 -> 5120 127 -> 78.
+struct Skinny {
+  int rt, s;        // row tiles per wave (0: not this form), k slices
+};
 
-extern "C" int helm_int8_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
-                              const void* scale, const void* bias, void* y, int64_t ldy, int M,
-                              int N, int K, void* stream) {
-  HELM_CHECK_ARG(x && q && scale && y, "helm_int8_gemm: null pointer");
-  HELM_CHECK_ARG(M >= 1 && N >= 1 && K >= 1, "helm_int8_gemm: M, N, K must be positive");
-  HELM_CHECK_ARG(ldx >= K && ldq >= K && ldy >= N, "helm_int8_gemm: leading dimension too small");
-  HELM_CHECK_SUPPORTED(K % BK == 0, "helm_int8_gemm: K must be a multiple of 64");
-  HELM_CHECK_SUPPORTED(ldq % 16 == 0 && ldx % 8 == 0, "helm_int8_gemm: row strides must be multiples of 16 (q) and 8 (x)");
-  HELM_CHECK_SUPPORTED(helm::aligned16(x) && helm::aligned16(q), "helm_int8_gemm: x and q must be 16-byte aligned");
+// workgroups per CU and ring stages of a tile height
+constexpr int skinny_occ(int rt) { return rt == 1 ? 4 : rt <= 3 ? 3 : 2; }
+constexpr int skinny_stages(int rt) { return rt == 1 ? 5 : rt == 3 ? 3 : 4; }
+
+Skinny pick_skinny(int M, int N, int K) {
+  Skinny p{0, 1};
+  const int mt = (M + 127) / 128;
+  const int rt = ((M + mt - 1) / mt + 31) / 32;
+  const int64_t tiles = (int64_t)mt * ((N + 63) / 64);
+  if (tiles > 512) return p;
+  p.rt = rt;
+  // k slices: rounds of workgroups x K-steps of a slice (0.4 us each, three for the
+  // start) against the partial sums' traffic (4 TB/s) and the second launch (3 us)
+  const int nk = K / BK;
+  const int64_t slots = 256 * skinny_occ(rt);
+  double best = -1.0;
+  for (int s = 1; s <= 32 && s <= std::max(1, nk / 4); ++s) {
+    const double rounds = (double)((tiles * s + slots - 1) / slots);
+    const double c = rounds * 0.4 * ((nk + s - 1) / s + 3) + (s > 1 ? 3.0 + (double)s * M * N * 8.0 / 4e6 : 0.0);
+    if (best < 0.0 || c < 0.97 * best) { best = c; p.s = s; }
+  }
+  // full-height tiles in one slice gain nothing over the prompt form's wider ones
+  // (100 x 5120 -> 17408 58.8 against 57.8 us, 200 x 4096 -> 12288 43.3 against 42.5)
+  if (rt == 4 && p.s == 1) p.rt = 0;
+  return p;
+}
+
+template <int RT>
+void launch_skinny(const Skinny& p, const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
+                   const void* scale, const void* bias, void* y, int64_t ldy, int M, int N, int K,
+                   float* part, hipStream_t s) {
+  constexpr int NS = skinny_stages(RT), OCC = skinny_occ(RT);
+  const dim3 grid((N + 63) / 64, (M + 32 * RT - 1) / (32 * RT), p.s);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, grid, dim3(kThreads), 0, s, static_cast<const uint16_t*>(x), ldx, q, ldq,
+                       static_cast<const uint16_t*>(scale), static_cast<const uint16_t*>(bias),
+                       static_cast<uint16_t*>(y), ldy, M, N, K, part);
+  };
+  if (p.s == 1) return go(int8_gemm_kernel<2, false, RT, NS, false, OCC>);
+  go(int8_gemm_kernel<2, false, RT, NS, true, OCC>);
+  const bool v4 = N % 4 == 0;
+  const int64_t n = (int64_t)M * N / (v4 ? 4 : 1);
+  const dim3 blocks((unsigned)((n + 255) / 256));
+  auto reduce = [&](auto kern) {
+    hipLaunchKernelGGL(kern, blocks, dim3(256), 0, s, part, p.s, static_cast<const uint16_t*>(scale),
+                       static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N);
+  };
+  if (v4) reduce(gemm_split_reduce_kernel<4>);
+  else reduce(gemm_split_reduce_kernel<1>);
+}
+
+int gemm_impl(const char* fn, const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
+              const void* scale, const void* bias, void* y, int64_t ldy, int M, int N, int K,
+              void* ws, int64_t ws_bytes, void* stream) {
+  const std::string f(fn);
+  HELM_CHECK_ARG(x && q && scale && y, f + ": null pointer");
+  HELM_CHECK_ARG(M >= 1 && N >= 1 && K >= 1, f + ": M, N, K must be positive");
+  HELM_CHECK_ARG(ldx >= K && ldq >= K && ldy >= N, f + ": leading dimension too small");
+  HELM_CHECK_SUPPORTED(K % BK == 0, f + ": K must be a multiple of 64");
+  HELM_CHECK_SUPPORTED(ldq % 16 == 0 && ldx % 8 == 0, f + ": row strides must be multiples of 16 (q) and 8 (x)");
+  HELM_CHECK_SUPPORTED(helm::aligned16(x) && helm::aligned16(q), f + ": x and q must be 16-byte aligned");
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  Skinny p = pick_skinny(M, N, K);
+  if (p.rt) {
+    if (!ws || !helm::aligned16(ws) || ws_bytes < (int64_t)p.s * M * N * (int64_t)sizeof(float)) {
+      p.s = 1;
+      if (p.rt == 4) p.rt = 0;
+    }
+  }
+  if (p.rt) {
+    float* part = static_cast<float*>(ws);
+    switch (p.rt) {
+      case 1: launch_skinny<1>(p, x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, part, s); break;
+      case 2: launch_skinny<2>(p, x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, part, s); break;
+      case 3: launch_skinny<3>(p, x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, part, s); break;
+      default: launch_skinny<4>(p, x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, part, s); break;
+    }
+    HELM_CHECK_LAUNCH(fn);
+    return HELM_OK;
+  }
   switch (pick_tn(M, N)) {
     case 2: launch_gemm<2>(x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, s); break;
     case 5: launch_gemm<5>(x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, s); break;
     default: launch_gemm<4>(x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, s); break;
   }
-  HELM_CHECK_LAUNCH("helm_int8_gemm launch");
+  HELM_CHECK_LAUNCH(fn);
   return HELM_OK;
+}
+
+}  // namespace
+
+extern "C" int helm_int8_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
+                              const void* scale, const void* bias, void* y, int64_t ldy, int M,
+                              int N, int K, void* stream) {
+  return gemm_impl("helm_int8_gemm", x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, nullptr, 0, stream);
+}
+
+extern "C" int64_t helm_int8_gemm_workspace_bytes(int M, int N, int K) {
+  if (M < 1 || N < 1 || K < BK) return 0;
+  const Skinny p = pick_skinny(M, N, K);
+  return p.rt && p.s > 1 ? (int64_t)p.s * M * N * (int64_t)sizeof(float) : 0;
+}
+
+extern "C" int helm_int8_gemm_ws(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
+                                 const void* scale, const void* bias, void* y, int64_t ldy, int M,
+                                 int N, int K, void* workspace, int64_t workspace_bytes, void* stream) {
+  return gemm_impl("helm_int8_gemm_ws", x, ldx, q, ldq, scale, bias, y, ldy, M, N, K, workspace,
+                   workspace_bytes, stream);
 }

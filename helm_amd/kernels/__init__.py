@@ -113,8 +113,11 @@ def int8_linear(input: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
                      qweight.stride(0), scale.data_ptr(), _native.ptr(bias), None, y2.data_ptr(),
                      y2.stride(0), M, N, K, _native.ptr(ws), ws_bytes, stream)
         return out
-    _native.call("helm_int8_gemm", x2.data_ptr(), x2.stride(0), qweight.data_ptr(), qweight.stride(0),
-                 scale.data_ptr(), _native.ptr(bias), y2.data_ptr(), y2.stride(0), M, N, K, stream)
+    ws_bytes = gemm_workspace_bytes(M, N, K)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=input.device) if ws_bytes else None
+    _native.call("helm_int8_gemm_ws", x2.data_ptr(), x2.stride(0), qweight.data_ptr(), qweight.stride(0),
+                 scale.data_ptr(), _native.ptr(bias), y2.data_ptr(), y2.stride(0), M, N, K,
+                 _native.ptr(ws), ws_bytes, stream)
     return out
 
 
@@ -130,6 +133,12 @@ def gemv_split_bytes(M: int, N: int, K: int) -> int:
     """Workspace with which helm_int8_gemv_ws takes its fastest form at this shape
     (0: none; at least gemv_workspace_bytes)."""
     return int(_native.lib().helm_int8_gemv_split_bytes(int(M), int(N), int(K)))
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_workspace_bytes(M: int, N: int, K: int) -> int:
+    """Workspace with which helm_int8_gemm_ws takes its fastest form (0: none)."""
+    return int(_native.lib().helm_int8_gemm_workspace_bytes(int(M), int(N), int(K)))
 
 
 def fp16_linear(input: torch.Tensor, weight: torch.Tensor,

@@ -122,6 +122,15 @@ int helm_int8_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
                    const void* scale, const void* bias, void* y, int64_t ldy,
                    int M, int N, int K, void* stream);
 
+/* helm_int8_gemm with a caller-owned workspace of helm_int8_gemm_workspace_bytes (0:
+ * none helps; 16-byte aligned, contents on entry do not matter): a few rows whose
+ * tiles leave CUs idle then split K over workgroups and add the fp32 partial sums
+ * in a second kernel.  Same results up to the fp32 summation order. */
+int64_t helm_int8_gemm_workspace_bytes(int M, int N, int K);
+int helm_int8_gemm_ws(const void* x, int64_t ldx, const int8_t* q, int64_t ldq,
+                      const void* scale, const void* bias, void* y, int64_t ldy, int M, int N, int K,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------ */
 /* Paged GQA decode attention                                               */
 /* ------------------------------------------------------------------------ */

@@ -618,3 +618,31 @@ def test_x_in_registers_fp16(M, N, K):
     wk[N // 2] = 0
     bound = (x.double().cpu().abs() @ wk.t()) * 2.0 ** -22 + exact.nan_to_num(0, 0, 0).abs() * 2.0 ** -11 + 2.0 ** -24
     assert ((y - exact).abs() <= bound)[:, keep].all()
+
+
+@pytest.mark.parametrize("M,N,K", [(17, 64, 64), (32, 1001, 256), (33, 4099, 1024), (64, 130, 4160), (77, 12288, 1088),
+                                   (97, 640, 5120), (128, 65, 17408), (150, 1000, 2048), (300, 5, 1280),
+                                   (513, 1024, 4096), (40, 25600, 512)])
+def test_int8_gemm_few_rows(M, N, K):
+    """The prefill GEMM's form for a few tiles of rows: every tile height, K of one
+    step, slices of unequal steps, odd N (scalar second pass), grids of one and two
+    rounds, with bias and a strided output; without the workspace the same rows."""
+    from helm_amd import _native
+    x, q, s, b = make_inputs(M, N, K, seed=M + N + K, bias=True)
+    xd, qd, sd, bd = to_dev(x, q, s, b)
+    exact = ol.int8_linear_exact(x, q, s, b)
+    bound = accumulation_bound(x, q, s)
+    assert_linear_ok(hk.int8_linear(xd, qd, sd, bd).cpu().numpy(), exact, f"M={M} N={N} K={K}", bound)
+    assert_linear_ok(hk.int8_linear(xd, qd, sd).cpu().numpy(), ol.int8_linear_exact(x, q, s), "no bias", bound)
+    stream = torch.cuda.current_stream().cuda_stream
+    out = torch.full((M, N + 3), float("nan"), dtype=torch.float16, device="cuda")
+    _native.call("helm_int8_gemm", xd.data_ptr(), K, qd.data_ptr(), K, sd.data_ptr(), bd.data_ptr(),
+                 out.data_ptr(), N + 3, M, N, K, stream)
+    assert_linear_ok(out[:, :N].cpu().numpy(), exact, "no workspace", bound)
+    need = _native.lib().helm_int8_gemm_workspace_bytes(M, N, K)
+    ws = torch.full((need // 4 + 4,), float("nan"), device="cuda")
+    out.fill_(float("nan"))
+    _native.call("helm_int8_gemm_ws", xd.data_ptr(), K, qd.data_ptr(), K, sd.data_ptr(), bd.data_ptr(),
+                 out.data_ptr(), N + 3, M, N, K, ws.data_ptr(), need, stream)
+    assert_linear_ok(out[:, :N].cpu().numpy(), exact, "strided output", bound)
+    assert torch.isnan(out[:, N:]).all()
