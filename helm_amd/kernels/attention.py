@@ -80,6 +80,22 @@ def choose_num_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: 
     return n
 
 
+def choose_batch_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: int = 16) -> int:
+    """Split count of one attention call over `batch` items whose lengths the host
+    does not know: with choose_num_splits the workgroups of the longest item are the
+    whole launch's tail while the short items' ones have ended.  From four items on
+    the count is doubled, from eight tripled (the CUs then take the longest item's
+    extra workgroups as the short ones end), to splits of at least 256 tokens.
+    Measured against choose_num_splits with lengths spread over 1/16 .. 1 of the
+    longest: 8 items of 12000 tokens 50.0 -> 33.9 us, 16 of 8000 65.0 -> 43.9, 4 of 4000
+    13.2 -> 11.6; the price where all are equal (more partials to merge): 63.9 -> 65.6,
+    83.8 -> 85.8, 15.0 -> 15.3.  Two or three items stay (two equal ones of 16384 25.3 ->
+    26.1 us), and four times as many splits cost equal lengths up to 15%."""
+    base = choose_num_splits(batch, num_kv_heads, max_pages, page_size)
+    more = 1 if batch < 4 else 2 if batch < 8 else 3
+    return max(base, min(more * base, max_pages * page_size // 256))
+
+
 def alloc_v(shape, dtype=torch.float16, device=None, pin_memory: bool = False,
             zero: bool = False) -> torch.Tensor:
     """V storage for `shape` = (..., T, D): allocated as (..., D, T) and returned as
@@ -288,7 +304,7 @@ def paged_decode_attention(q: torch.Tensor, pool: PoolView, page_table: torch.Te
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     if num_splits is None:
-        num_splits = choose_num_splits(B, pool.num_kv_heads, page_table.shape[1], page_size)
+        num_splits = choose_batch_splits(B, pool.num_kv_heads, page_table.shape[1], page_size)
     ws = workspace if workspace is not None else AttnWorkspace(q.device)
     part_o, part_ml = ws.get(B, Hq, D, num_splits)
     paged_decode_attention_partial(q, pool, page_table, seq_lens, page_size, scale, part_o,
