@@ -236,16 +236,13 @@ __global__ __launch_bounds__(kThreads, OCC) void int8_gemm_kernel(
 #pragma unroll
   for (int i = 0; i < NS - 1; ++i)
     if (i < nk) copy(i, i);
-  int st = 0, fill = NS - 1;
   for (int kb = 0; kb < nk; ++kb) {
     if (kb + NS - 2 < nk) wait_vm<(NS - 2) * C::kCopiesMin>();
     else wait_vm<0>();
     lds_read_barrier();
-    if (kb + NS - 1 < nk) copy(kb + NS - 1, fill);
-    if constexpr (KSPLIT) compute_ks(st);
-    else compute(st);
-    st = st + 1 == NS ? 0 : st + 1;
-    fill = fill + 1 == NS ? 0 : fill + 1;
+    if (kb + NS - 1 < nk) copy(kb + NS - 1, (kb + NS - 1) % NS);
+    if constexpr (KSPLIT) compute_ks(kb % NS);
+    else compute(kb % NS);
   }
 
   if constexpr (KSPLIT) {

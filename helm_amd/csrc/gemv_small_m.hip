@@ -1,5 +1,9 @@
 // gemv_small_m.hip — INT8 weight-only linear for 3 <= M <= 16 tokens.
 //
+// Reached for K = 4096, for long K whose 16-row tiles fill the CUs in one round, for
+// calls without the workspace that gemv_xreg.hip needs for long K, and (fp16 weights)
+// for K below 2048 or beyond 5120; gemv_xreg.hip takes the rest.
+//
 // Same contract as the decode GEMV (y = fp16(s * (x . q^T) + bias), fp32
 // accumulation; optional residual add), for a few tokens at once (small-batch
 // or multi-token decode).  With M tokens every weight byte feeds M products, so
@@ -184,7 +188,7 @@ __global__ __launch_bounds__(W * 64) void int8_small_m_kernel(SmallMArgs a) {
 
 // ---------------------------------------------------------------------------
 // Resident form (used for K = 4096, and K = 12288 up to 4 tokens; the ring form
-// above serves every other shape).  Reading x^T from L2 for every 16-row tile
+// above serves the rest).  Reading x^T from L2 for every 16-row tile
 // costs more than the weights themselves (at 4096 -> 12288 with 16 tokens:
 // 19.4 us with the operand loads from L2, 11.0 us with the same operands read
 // from LDS; with 4 tokens 13.8 vs 10.5 us), so here x^T stays in LDS:

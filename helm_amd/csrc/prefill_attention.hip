@@ -15,21 +15,24 @@
 // A workgroup is one kv head x a block of 4 * 16 * NC rows, one wave per 16 * NC
 // of them; rows are (query, head of the group) pairs, query-major, so a few
 // queries fill a block with all their heads (17 queries of a group of 4: one
-// block, not four) and a block spans fewer positions of the diagonal.  The four waves need the same K/V tiles, so the workgroup
-// fetches each 32-key tile once, straight into LDS (global_load_lds_dwordx4:
-// every lane moves 16 bytes, a wave 1 KiB of contiguous pool memory), double
-// buffered: tile s+1 is copied while tile s is computed, and the waves read
-// their MFMA operands from LDS.  The copy of tile s+1 goes out right after the
-// barrier of step s, from page slots looked up a step earlier, ahead of the operand
-// reads of tile s (a compiler-tracked copy would make those reads wait for it).
-// A step is a serial chain of about 2000 cycles (operand reads, QK, softmax, PV);
-// 64 KB of LDS operand reads per step, 512 cycles of MFMA per wave and about as many of VALU
-// work bound it, two workgroups per CU overlap.  Measured: 14B heads at T =
-// 2048 74.5 -> 67.1 us (641 TFLOP/s), 32 heads, 390 queries over 7000 cached keys
-// (104 workgroups, five key splits) 198 -> 84 us, T = 4096 over 12000 keys 1305 -> 1221 us
-// (966 TFLOP/s), left-padding mask at T = 2048 171 -> 151 us.
-// LDS layouts (16-byte chunks) are chosen so
-// that both the copies and the operand reads are conflict free:
+// block, not four) and a block spans fewer positions of the diagonal.  The four
+// waves need the same K/V tiles, so the workgroup fetches each 32-key tile once,
+// straight into LDS (global_load_lds_dwordx4: every lane moves 16 bytes, a wave 1
+// KiB of contiguous pool memory), double buffered: tile s+1 is copied while tile s
+// is computed, and the waves read their MFMA operands from LDS.  The copy of tile
+// s+1 goes out right after the barrier of step s, from page slots looked up a step
+// earlier, ahead of the operand reads of tile s (a compiler-tracked copy would make
+// those reads wait for it).
+//
+// A step is a serial chain of about 2000 cycles (operand reads, QK, softmax, PV); per
+// step 64 KB of LDS reads a workgroup, 512 cycles of MFMA a wave and about as many
+// of VALU work bound it, two workgroups per CU overlap.  Measured: 14B heads at T =
+// 2048 74.5 -> 67.1 us (641 TFLOP/s), 390 queries of 32 heads over 7000 cached keys
+// (104 workgroups, four key splits) 198 -> 84 us, T = 4096 over 12000 keys 1305 -> 1221
+// us (966 TFLOP/s), left-padding mask at T = 2048 171 -> 151 us.
+//
+// LDS layouts (16-byte chunks) are chosen so that both the copies and the operand
+// reads are conflict free:
 //   K: row-major [32 keys][D/8 chunks], chunk index XOR-swizzled by key bits
 //      {0,1,3,4}, so the 16 rows one operand read touches hit 16 distinct banks;
 //   V: [D/16 dim groups][4 key chunks][16 dims] — one operand read is 16

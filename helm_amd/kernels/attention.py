@@ -14,6 +14,7 @@ the strides the kernels need (see helm_kv_pool in include/helm_mi355x.h).
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 from typing import Optional, Tuple
@@ -80,6 +81,7 @@ def choose_num_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: 
     return n
 
 
+@functools.lru_cache(maxsize=4096)
 def choose_batch_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: int = 16) -> int:
     """Split count of one attention call over `batch` items whose lengths the host
     does not know: with choose_num_splits the workgroups of the longest item are the
@@ -418,6 +420,12 @@ def kernel_mask(mask: torch.Tensor, T: int, kv_len: int, Hq: int):
     return m, (0 if mask.shape[0] == 1 else T * pitch), key_end
 
 
+@functools.lru_cache(maxsize=4096)
+def prefill_workspace_bytes(T: int, q_start: int, Hq: int, Hkv: int, D: int) -> int:
+    """Workspace with which helm_prefill_attn_ws takes its fastest form (0: none)."""
+    return int(_native.lib().helm_prefill_attn_workspace_bytes(T, q_start, Hq, Hkv, D))
+
+
 def prefill_attention(q: torch.Tensor, pool: PoolView, page_table: torch.Tensor, page_size: int,
                       q_start: int = 0, scale: Optional[float] = None,
                       out: Optional[torch.Tensor] = None,
@@ -446,8 +454,7 @@ def prefill_attention(q: torch.Tensor, pool: PoolView, page_table: torch.Tensor,
     if out is None:
         out = torch.empty(T, Hq, D, dtype=torch.float16, device=q.device)
     if mask is None:
-        need = int(_native.lib().helm_prefill_attn_workspace_bytes(T, int(q_start), Hq,
-                                                                   pool.num_kv_heads, D))
+        need = prefill_workspace_bytes(T, int(q_start), Hq, pool.num_kv_heads, D)
         ws = torch.empty(need, dtype=torch.uint8, device=q.device) if need else None
         _native.call("helm_prefill_attn_ws", q.data_ptr(), q.stride(0), q.stride(1), pool.c_ref(),
                      page_table.data_ptr(), int(q_start), T, Hq, pool.num_kv_heads, D, page_size,

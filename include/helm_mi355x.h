@@ -90,8 +90,9 @@ int helm_int8_gemv_fused(const void* x, int64_t ldx, const void* norm_w, float e
  * on entry do not matter).  Shapes whose activations of 8-16 tokens exceed the
  * kernel's LDS (K a multiple of 3072 above 4096, N % 4 == 0, e.g. the Qwen3-8B
  * down projection 12288 -> 4096) then split K over workgroups, keep fp32 partial
- * sums there and reduce them in a second kernel; every other shape (workspace
- * bytes 0) runs as helm_int8_gemv_fused and may pass workspace NULL.  Same results
+ * sums there and reduce them in a second kernel; every other shape may pass
+ * workspace NULL and then runs as helm_int8_gemv_fused, or
+ * helm_int8_gemv_split_bytes of workspace for the split form of other long K.  Same results
  * up to the fp32 summation order.  Replaces the same decode fast path as
  * helm_int8_gemv (helm/kernels/fp16_gemv.cpp:105-157). */
 int64_t helm_int8_gemv_workspace_bytes(int M, int N, int K);
