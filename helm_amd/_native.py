@@ -136,7 +136,9 @@ def call(name: str, *args) -> None:
     f = _bound.get(name)
     if f is None:
         f = _bound[name] = getattr(lib(), name)
-    check(f(*args))
+    rc = f(*args)
+    if rc != 0:
+        check(rc)
 
 
 def version() -> str:
@@ -163,7 +165,7 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 def require_cuda(*tensors: Optional[torch.Tensor], what: str = "helm_amd") -> None:
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise RuntimeError(f"{what}: tensors must be on the GPU (got {t.device}); "
                                "this library has no CPU path")
 

@@ -73,7 +73,7 @@ def dequantize(qweight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
 def _flatten(x: torch.Tensor, K: int, what: str) -> torch.Tensor:
     if x.shape[-1] != K:
         raise RuntimeError(f"{what}: input last dim ({x.shape[-1]}) != weight K ({K})")
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, K)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
         x2 = x2.contiguous()
     return x2
@@ -99,15 +99,15 @@ def int8_linear(input: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
         raise RuntimeError("int8_linear: bias must be fp16 [N]")
     x2 = _flatten(input, K, "int8_linear")
     M = x2.shape[0]
-    lead = input.shape[:-1]
     if out is None:
-        out = torch.empty(*lead, N, dtype=torch.float16, device=input.device)
-    y2 = out.view(-1, N)
+        out = torch.empty((*input.shape[:-1], N), dtype=torch.float16, device=input.device)
+    y2 = out if out.dim() == 2 and out.shape[1] == N else out.view(-1, N)
     if M == 0:
         return out
     stream = _native.stream_ptr(input.device)
     if M <= GEMV_MAX_TOKENS:
-        ws_bytes = gemv_split_bytes(M, N, K)
+        # (one or two tokens never split)
+        ws_bytes = gemv_split_bytes(M, N, K) if M > 2 else 0
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=input.device) if ws_bytes else None
         _native.call("helm_int8_gemv_ws", x2.data_ptr(), x2.stride(0), qweight.data_ptr(),
                      qweight.stride(0), scale.data_ptr(), _native.ptr(bias), None, y2.data_ptr(),
