@@ -347,16 +347,18 @@ void launch_gemm(const void* x, int64_t ldx, const int8_t* q, int64_t ldq, const
                        static_cast<const uint16_t*>(bias), static_cast<uint16_t*>(y), ldy, M, N, K, nullptr);
 }
 
+// Tile width of the prompt form that HELM_GEMM_TN asks for (for every shape), or 0.
 int env_tn() {
   const char* v = getenv("HELM_GEMM_TN");
-  return v ? atoi(v) : 0;
+  const int tn = v ? atoi(v) : 0;
+  return tn == 2 || tn == 4 || tn == 5 ? tn : 0;
 }
 
 // Tile width: the N extent per workgroup that fills the GPU's 2 x 256 workgroup
 // slots most evenly (two workgroups fit per CU), wider tiles preferred on ties.
 int pick_tn(int M, int N) {
   const int env = env_tn();
-  if (env == 2 || env == 4 || env == 5) return env;
+  if (env) return env;
   const int mt = (M + BM - 1) / BM;
   int best = 4;
   double best_eff = -1.0;
@@ -450,7 +452,7 @@ int gemm_impl(const char* fn, const void* x, int64_t ldx, const int8_t* q, int64
   HELM_CHECK_SUPPORTED(ldq % 16 == 0 && ldx % 8 == 0, f + ": row strides must be multiples of 16 (q) and 8 (x)");
   HELM_CHECK_SUPPORTED(helm::aligned16(x) && helm::aligned16(q), f + ": x and q must be 16-byte aligned");
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  Skinny p = pick_skinny(M, N, K);
+  Skinny p = env_tn() ? Skinny{0, 1} : pick_skinny(M, N, K);
   if (p.rt) {
     if (!ws || !helm::aligned16(ws) || ws_bytes < (int64_t)p.s * M * N * (int64_t)sizeof(float)) {
       p.s = 1;
