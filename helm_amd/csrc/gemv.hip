@@ -768,15 +768,32 @@ extern "C" int helm_int8_gemv(const void* x, int64_t ldx, const int8_t* q, int64
 }
 
 // fp16 weights at 3-16 tokens on the matrix cores; false when neither form takes
-// the shape.  x^T in registers from K = 2048 on (4096 -> 151936 at 4 / 16 tokens 233
-// -> 195 and 246 -> 211 us; 5120 at 16 tokens, whose x rows exceed LDS, 1058 -> 260),
-// x^T in LDS below (1024 -> 151936 at 8 tokens 54.4 against 55.4 us).
+// the shape.  us at 8 tokens with the norm, weights rotating through HBM:
+//   x^T in registers walks whole units at K = 2048, 4096 and 5120: 4096 -> 151936 194
+//   against 228 with x^T in LDS, 4096 -> 4096 12 against 27, 2048 -> 32000 25.4 against
+//   28.8, 5120 -> 8192 20 against 36; from about 65000 outputs on the two meet at 5120
+//   (107 against 105 at 65536, 244 against 234 at 151936).
+//   At other K it copies more units than there are (2560: 64 for 40), and the form
+//   with x^T in LDS is the faster from the number of outputs on that fills its
+//   workgroups of 128 rows: 2560 -> 151936 120 against 169, 3072 -> 49152 53 against 62,
+//   but 2560 -> 8192 20 against 15.6; the two meet near 13000 outputs at 2304 and
+//   2560, 16384 at 3072, 20000 at 3584 and 4608.
+//   Below 2048 x^T in LDS (1024 -> 32000 13.4 without the norm, 13.9 in registers).
+//   Three tokens (registers or the streaming kernel): up to 4096 rows of K in 2560 ..
+//   4096 the norm prologue of one row tile per workgroup costs more than the
+//   streaming kernel's (4096 -> 4096 11.4 against 10.1; 8192 outputs 15.6 against 16.0).
 static bool fp16_matrix_form(const void* x, int64_t ldx, const void* norm_w, float eps,
                              const void* w, int64_t ldw, const void* bias, void* y, int64_t ldy,
                              int M, int N, int K, hipStream_t s) {
   auto lds = [&] { return helm::launch_fp16_small_m(x, ldx, norm_w, eps, w, ldw, bias, y, ldy, M, N, K, s); };
   auto xreg = [&] { return helm::launch_xreg_fp16(x, ldx, norm_w, eps, w, ldw, bias, y, ldy, M, N, K, s); };
-  return K < 2048 ? (lds() || xreg()) : (xreg() || lds());
+  if (M == 3 && norm_w && N <= 4096 && K > 2048 && K <= 4096) return false;
+  const int units = (K + 63) / 64, walked = helm::xreg_fp16_units(K);
+  bool lds_first;
+  if (K < 2048) lds_first = true;
+  else if (units == walked) lds_first = K > 4096 && N > 65536;
+  else lds_first = N > (4 * units <= 3 * walked ? 14336 : 20480);
+  return lds_first ? (lds() || xreg()) : (xreg() || lds());
 }
 
 extern "C" int helm_fp16_gemv(const void* x, int64_t ldx, const void* w, int64_t ldw,

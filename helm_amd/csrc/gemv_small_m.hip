@@ -2,7 +2,8 @@
 //
 // Reached for K = 4096, for long K whose 16-row tiles fill the CUs in one round, for
 // calls without the workspace that gemv_xreg.hip needs for long K, and (fp16 weights)
-// for K below 2048 or beyond 5120; gemv_xreg.hip takes the rest.
+// for K below 2048 or beyond 5120 and for many outputs at K whose units
+// gemv_xreg.hip does not walk whole; gemv_xreg.hip takes the rest.
 //
 // Same contract as the decode GEMV (y = fp16(s * (x . q^T) + bias), fp32
 // accumulation; optional residual add), for a few tokens at once (small-batch
@@ -818,8 +819,7 @@ bool launch_int8_small_m(const void* x, int64_t ldx, const void* norm_w, float e
 // is not one it takes (K % 128 != 0, x rows beyond LDS, weights above 2 GiB,
 // unaligned operands).  Qwen3-8B lm_head (151936 x 4096, fused norm): 8 tokens
 // 386 -> 231 us, 16 tokens 882 -> 244 us, 4 tokens 249 -> 231 us against the
-// tiled / streaming dot-product kernels; at 3 tokens the streaming kernel stays
-// (216-226 against 233 us).
+// tiled / streaming dot-product kernels (three tokens: gemv_xreg.hip, or streaming).
 bool launch_fp16_small_m(const void* x, int64_t ldx, const void* norm_w, float eps,
                          const void* w, int64_t ldw, const void* bias, void* y, int64_t ldy,
                          int M, int N, int K, hipStream_t stream) {

@@ -505,12 +505,20 @@ bool launch_xreg_swiglu(const void* x, int64_t ldx, const void* norm_w, float ep
   return true;
 }
 
+// Units of 64 k the fp16 form walks at this K: its eight waves walk 2, 4, 8 or 10
+// each, whole K or not (the products of units past K are left out, their copies are
+// not).  0: beyond its registers.
+int xreg_fp16_units(int K) {
+  const int uw = uw_of(units_of(K, false), 1);
+  return uw > kMaxUwF16 ? 0 : kW * (uw <= 2 ? 2 : uw <= 4 ? 4 : uw <= 8 ? 8 : kMaxUwF16);
+}
+
 bool launch_xreg_fp16(const void* x, int64_t ldx, const void* norm_w, float eps, const void* w,
                       int64_t ldw, const void* bias, void* y, int64_t ldy, int M, int N, int K,
                       hipStream_t stream) {
   if (!common_ok(x, ldx, norm_w, w, ldw * 2, M, N) || K % 64 != 0) return false;   // whole units
-  const int uw = uw_of(units_of(K, false), 1);
-  if (uw > kMaxUwF16) return false;
+  const int uw = xreg_fp16_units(K) / kW;
+  if (!uw) return false;
   XregArgs a{};
   a.x = static_cast<const uint16_t*>(x); a.ldx = ldx;
   a.norm_w = static_cast<const uint16_t*>(norm_w); a.eps = eps;
@@ -518,9 +526,9 @@ bool launch_xreg_fp16(const void* x, int64_t ldx, const void* norm_w, float eps,
   a.bias = static_cast<const uint16_t*>(bias);
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.S = 1;
-  if (uw <= 2) launch_f16<2>(a, stream);
-  else if (uw <= 4) launch_f16<4>(a, stream);
-  else if (uw <= 8) launch_f16<8>(a, stream);
+  if (uw == 2) launch_f16<2>(a, stream);
+  else if (uw == 4) launch_f16<4>(a, stream);
+  else if (uw == 8) launch_f16<8>(a, stream);
   else launch_f16<10>(a, stream);
   return true;
 }

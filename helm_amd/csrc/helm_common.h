@@ -67,6 +67,7 @@ bool launch_xreg_swiglu(const void* x, int64_t ldx, const void* norm_w, float ep
                         const int8_t* q_gate, const void* s_gate, const int8_t* q_up,
                         const void* s_up, int64_t ldq, void* y, int64_t ldy, int M, int N, int K,
                         hipStream_t stream);
+int xreg_fp16_units(int K);
 bool launch_xreg_fp16(const void* x, int64_t ldx, const void* norm_w, float eps, const void* w,
                       int64_t ldw, const void* bias, void* y, int64_t ldy, int M, int N, int K,
                       hipStream_t stream);

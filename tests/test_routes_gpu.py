@@ -7,6 +7,7 @@ import torch
 from torch.profiler import ProfilerActivity, profile
 
 from helm_amd import kernels as hk
+from helm_amd.kernels import fused
 
 pytestmark = pytest.mark.gpu
 
@@ -44,3 +45,40 @@ def test_gemm_tile_width_override(M, N, K, tn, monkeypatch, tmp_path):
     monkeypatch.setenv("HELM_GEMM_TN", str(tn))
     (name, _), = launches(lambda: hk.int8_linear(x, q, s), tmp_path)
     assert name.startswith(f"int8_gemm_kernel<{tn}, {'true' if tn >= 4 else 'false'}, 4, 3, false"), name
+
+
+LDS, REGS, STREAM = "fp16_small_m_kernel<", "xreg_gemv_kernel<false", "gemv_stream_kernel<"
+
+
+@pytest.mark.parametrize("M,N,K,norm,kernel", [
+    (8, 14336, 2560, True, REGS), (8, 14337, 2560, True, LDS), (4, 14337, 3072, False, LDS),
+    (4, 20480, 3584, True, REGS), (13, 20481, 3584, False, LDS), (5, 20481, 4608, True, LDS),
+    (16, 20481, 4608, True, REGS),          # its x rows exceed LDS
+    (8, 32000, 4096, True, REGS), (8, 32000, 2048, False, REGS),
+    (5, 65536, 5120, False, REGS), (12, 65537, 5120, True, LDS), (16, 65537, 5120, True, REGS),
+    (4, 5000, 1920, True, LDS), (3, 5000, 1920, True, REGS),
+    (3, 4096, 2560, True, STREAM), (3, 4097, 2560, True, REGS), (3, 4096, 2560, False, REGS),
+    (3, 4096, 4096, True, STREAM), (3, 4096, 5120, True, REGS)])
+def test_fp16_form_by_size(M, N, K, norm, kernel, tmp_path):
+    """Either side of each line of the rule for fp16 weights, and the result there
+    (fp32 accumulation and one rounding; with the norm one step of an fp16 operand
+    more)."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    w = (torch.randn(N, K, generator=g, device="cuda") * 0.02).half()
+    nw = (1 + 0.1 * torch.randn(K, generator=g, device="cuda")).half()
+    run = (lambda: fused.fp16_gemv_rmsnorm(x, nw, 1e-6, w)) if norm else (lambda: hk.fp16_linear(x, w))
+    (name, _), = launches(run, tmp_path)
+    assert name.startswith(kernel), name
+    rows = torch.randperm(N, generator=g, device="cuda")[:4000]
+    rows[0], rows[1] = N - 1, 0
+    xn = x.float()
+    if norm:
+        xn = (nw.float() * (xn * torch.rsqrt(xn.square().mean(-1, keepdim=True) + 1e-6)).half().float()).half()
+    ws = w[rows].double().t().contiguous()
+    exact = torch.mm(xn.double(), ws)
+    mag = torch.mm(xn.double().abs(), ws.abs())
+    bound = mag * 2.0 ** -22 + exact.abs() * 2.0 ** -11 + 2.0 ** -24
+    if norm:      # x * rsqrt may round to the neighbouring fp16 value
+        bound += mag * 2.0 ** -10
+    assert ((run()[:, rows].double() - exact).abs() <= bound).all()
