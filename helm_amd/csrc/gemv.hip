@@ -672,6 +672,48 @@ int check_common(const void* x, int64_t ldx, const void* w, int64_t ldw, const v
   return HELM_OK;
 }
 
+// int8 at 3-16 tokens: whether the form of one 16-row tile per workgroup and round
+// (gemv_small_m.hip: x^T in LDS, or streamed from L2 by its ring) goes first, else x^T
+// in registers, persistent over the tiles (gemv_xreg.hip).  x in registers is the
+// faster wherever the tiles leave a last round of the 256 CUs part empty (17408 -> 5120
+// at 8 tokens 34.4 -> 23.9 us, 5120 -> 17408 29.6 -> 19.9, 8192 -> 5120 18.4 -> 13.8) and
+// for K up to 6144 nearly everywhere; the tile form where its grid is whole rounds.
+// us, tile form against registers, weights rotating through HBM:
+//   K = 4096: 4096 -> 12288 at 16 tokens 12.2 / 14.9, 4096 -> 4096 7.4 / 9.2;
+//   K = 2048, one round, 12-16 tokens: 2048 -> 2048 5.5 / 5.8;
+//   k slices of 3072 (8-16 tokens, 64-row groups x slices the grid) in one round of
+//     workgroups, where the busiest wave of the other form walks 10 units or more
+//     (12288 -> 4096 at 8 14.8 / 16.6, 24576 -> 2048 15.8 / 17.2, 9216 -> 4096 13.9 /
+//     14.8; with 9 units 12288 -> 3072 14.4 / 13.4, 9216 -> 4000 14.0 / 12.9); 6144
+//     needs no slices in registers: only the whole round, 6144 -> 8192 at 16 15.1 / 16.2;
+//   K = 12288, up to 4 tokens (all of x^T in LDS): 12288 -> 4096 11.4 / 15.5, 12288 ->
+//     1536 9.2 / 11.4, 12288 -> 6144 18.1 / 19.2, but 12288 -> 5120 17.5 / 16.5;
+//   other K from 6144 on, ring, tiles of one round: 8192 -> 4096 at 8 tokens 11.3 / 13.6
+//     and at 16 13.4 / 15.4, 14336 -> 4096 at 8 17.2 / 17.9 but at 14 19.8 / 19.0, 18432 ->
+//     4096 at 4 18.9 / 20.2, 6144 -> 4096 at 6 9.2 / 9.5 (at 8 12.7 / 10.2);
+//     three quarters of a round 8192 -> 3072 at 6 10.1 / 10.9, 16384 -> 3072 at 4
+//     15.2 / 16.4 (15360 -> 3072, whose ring has four waves instead of eight, 16.5 / 14.9);
+//     half a round 8192 -> 2048 at 4 9.6 / 10.3; two rounds 7168 -> 8192 at 12 16.2 / 18.3,
+//     but 10240 -> 8192 22.5 / 21.8.
+bool tile_form_first(int M, int N, int K, int64_t part_bytes) {
+  const int tiles = (N + 15) / 16;
+  const bool round1 = tiles > 208 && tiles <= 256, round2 = tiles > 480 && tiles <= 512;
+  if (K == 4096) return true;
+  if (K == 2048) return M >= 12 && tiles <= 256;
+  if (K < 6144) return false;
+  const int64_t ws = helm::int8_small_m_workspace_bytes(M, N, K);
+  if (ws > 0 && part_bytes >= ws) {
+    const int64_t grid = (int64_t)((N + 63) / 64) * (K / 3072);
+    return K == 6144 ? M >= 12 && grid == 256 : grid <= 256 && helm::xreg_walk_units(N, K) >= 10;
+  }
+  if (K == 6144) return M < 8 && round1;
+  if (K == 12288 && M <= 4) return (tiles > 64 && tiles <= 256) || (tiles > 352 && tiles <= 512);
+  const int most = K <= 8192 ? 16 : K <= 16384 ? 10 : 7;    // tokens
+  if (round1) return M <= most;
+  if (tiles > 176 && tiles <= 208) return M <= (K <= 8192 ? 8 : K <= 16384 && K % 2048 == 0 ? 4 : 0);
+  return K <= 8192 && (round2 || (M <= 6 && tiles > 95 && tiles <= 128));
+}
+
 }  // namespace
 
 // The int8 decode linear behind helm_int8_gemv, _fused and _ws: `part` null, or a
@@ -694,17 +736,8 @@ static int int8_gemv_impl(const void* x, int64_t ldx, const void* norm_w, float 
   a.y = static_cast<uint16_t*>(y); a.ldy = ldy;
   a.M = M; a.N = N; a.K = K; a.kt = choose_kt(M, K);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // 3-16 tokens, two matrix-core forms.  One 16-row tile per workgroup with x^T in
-  // LDS (gemv_small_m.hip) where its grid is whole and x fits: K = 4096 (4096 ->
-  // 12288 at 16 tokens 12.2 against 14.9 us, 4096 -> 4096 7.4 against 9.2), and K of
-  // 6145-16384 whose row tiles fill the 256 CUs in one round (12288 -> 4096 at 8
-  // tokens 14.8 against 16.8 us; at 8-16 tokens only as its split form).  Elsewhere
-  // x^T in registers, persistent over the row tiles (gemv_xreg.hip): 17408 -> 5120
-  // at 8 tokens 34.4 -> 23.9 us, 12288 -> 5120 20.5 -> 17.4, 5120 -> 17408 29.6 ->
-  // 19.9, 6144 -> 4096 13.6 -> 10.5.
-  const int tiles = (N + 15) / 16;
-  const bool tile_form = K == 4096 || (K > 6144 && K <= 16384 && tiles > 224 && tiles <= 256 &&
-                                       (M < 8 || K % 3072 == 0));
+  // 3-16 tokens, two matrix-core forms: tile_form_first
+  const bool tile_form = tile_form_first(M, N, K, part_bytes);
   auto tile = [&] {
     return helm::launch_int8_small_m(x, ldx, norm_w, eps, q, ldq, scale, bias, residual, y, ldy, M, N,
                                      K, part, part_bytes, s);

@@ -375,6 +375,12 @@ int uw_of(int units, int S) {
   return (sn + kW - 1) / kW;
 }
 
+// Ring units the busiest wave walks with S slices: rounds of row tiles x units of a wave.
+int64_t walk_of(int N, int units, int S) {
+  const int tiles = (N + 15) / 16, nb = std::max(1, kCUs / S);
+  return (int64_t)((tiles + nb - 1) / nb) * uw_of(units, S);
+}
+
 // k slices for K that one slice does not hold: of the few smallest counts the one
 // whose busiest workgroup walks the fewest ring units (rounds of row tiles x units
 // per wave, unfilled ones included: they take ring slots too).  More slices than
@@ -384,14 +390,9 @@ int choose_slices(int N, int units) {
   int s0 = 1;
   while (uw_of(units, s0) > kMaxUwI8) ++s0;
   if (s0 == 1) return 1;
-  const int tiles = (N + 15) / 16;
   int best = s0;
-  int64_t best_cost = -1;
-  for (int s = s0; s < s0 + 4; ++s) {
-    const int nb = std::max(1, kCUs / s);
-    const int64_t cost = (int64_t)((tiles + nb - 1) / nb) * uw_of(units, s);
-    if (best_cost < 0 || cost < best_cost) { best_cost = cost; best = s; }
-  }
+  for (int s = s0 + 1; s < s0 + 4; ++s)
+    if (walk_of(N, units, s) < walk_of(N, units, best)) best = s;
   return best;
 }
 
@@ -449,6 +450,12 @@ bool common_ok(const void* x, int64_t ldx, const void* norm_w, const void* w, in
 }  // namespace
 
 namespace helm {
+
+// Ring units (128 bytes of 16 rows) the busiest wave walks in the int8 form.
+int xreg_walk_units(int N, int K) {
+  const int units = units_of(K, true);
+  return (int)std::min<int64_t>(walk_of(N, units, choose_slices(N, units)), 1 << 30);
+}
 
 int64_t xreg_workspace_bytes(int M, int N, int K) {
   if (M < 3 || M > 16 || N < 1 || K < 16 || K % 16 != 0) return 0;

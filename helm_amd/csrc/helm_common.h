@@ -59,6 +59,7 @@ bool launch_fp16_small_m(const void* x, int64_t ldx, const void* norm_w, float e
 // The same three for 3 <= M <= 16 tokens with x^T in registers (gemv_xreg.hip);
 // int8 K beyond one k slice needs xreg_workspace_bytes of `part`.
 int64_t xreg_workspace_bytes(int M, int N, int K);
+int xreg_walk_units(int N, int K);
 bool launch_xreg_int8(const void* x, int64_t ldx, const void* norm_w, float eps, const int8_t* q,
                       int64_t ldq, const void* scale, const void* bias, const void* residual,
                       void* y, int64_t ldy, int M, int N, int K, float* part, int64_t part_bytes,

@@ -82,3 +82,40 @@ def test_fp16_form_by_size(M, N, K, norm, kernel, tmp_path):
     if norm:      # x * rsqrt may round to the neighbouring fp16 value
         bound += mag * 2.0 ** -10
     assert ((run()[:, rows].double() - exact).abs() <= bound).all()
+
+
+RES, RING, REG8 = "int8_small_m_resident_kernel<", "int8_small_m_kernel<", "xreg_gemv_kernel<true"
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [
+    (3, 1000, 4096, RES), (16, 4097, 4096, RES),
+    (11, 2048, 2048, REG8), (12, 4096, 2048, RING), (12, 4097, 2048, REG8),
+    (7, 4096, 6144, RING), (8, 4096, 6144, REG8), (7, 3328, 6144, REG8), (7, 4097, 6144, REG8),
+    (12, 8192, 6144, RES), (11, 8192, 6144, REG8), (12, 8128, 6144, REG8),
+    # k slices of 3072 in one round of workgroups, the other form walking 10 units or more
+    (8, 4096, 9216, RES), (8, 4000, 9216, REG8), (12, 4096, 12288, RES), (12, 4092, 12288, RES),
+    (16, 3844, 12288, RES), (9, 3072, 12288, REG8), (9, 4100, 12288, REG8), (8, 2048, 24576, RES),
+    (12, 3072, 15360, RES), (12, 4092, 15360, REG8), (8, 4098, 12288, REG8),
+    # all of x^T in LDS
+    (4, 1040, 12288, RES), (4, 1024, 12288, REG8), (3, 5120, 12288, REG8), (4, 8192, 12288, RES),
+    # ring
+    (16, 4096, 8192, RING), (16, 4097, 8192, REG8), (16, 3344, 7168, RING), (9, 3328, 8192, REG8),
+    (8, 3328, 8192, RING), (6, 2048, 8192, RING), (7, 2048, 8192, REG8), (10, 8192, 7168, RING),
+    (10, 4096, 14336, RING), (11, 4096, 14336, REG8), (4, 3072, 16384, RING), (5, 3072, 16384, REG8),
+    (4, 3072, 15360, REG8), (7, 4096, 17408, RING), (8, 4096, 17408, REG8), (8, 5120, 17408, REG8)])
+def test_int8_form_by_size(M, N, K, kernel, tmp_path):
+    """Either side of each line of the rule for int8 weights at 3-16 tokens, and the
+    result there (exact products, fp32 accumulation, one rounding)."""
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device="cuda").half()
+    q = torch.randint(-127, 128, (N, K), dtype=torch.int8, generator=g, device="cuda")
+    s = (torch.rand(N, generator=g, device="cuda") * 1e-2).half()
+    seen = launches(lambda: hk.int8_linear(x, q, s), tmp_path)
+    assert seen[0][0].startswith(kernel), seen
+    if kernel == RES and K != 4096 and M >= 8:
+        assert seen[1][0].startswith("small_m_split_reduce_kernel"), seen
+    qs = q.double().t().contiguous()
+    exact = torch.mm(x.double(), qs) * s.double()
+    mag = torch.mm(x.double().abs(), qs.abs()) * s.double()
+    bound = mag * 2.0 ** -22 + exact.abs() * 2.0 ** -11 + 2.0 ** -24
+    assert ((hk.int8_linear(x, q, s).double() - exact).abs() <= bound).all()
