@@ -154,10 +154,14 @@ __global__ __launch_bounds__(256) void qk_norm_rope_append_kernel(
 // tokens, 64 + 16 heads: 123 -> 35.7 us (4.7 TB/s).
 constexpr int kTT = 16;       // tokens of a workgroup
 constexpr int kHC = 8;        // heads of a workgroup
-// fewest tokens: a workgroup's chain (factors, then four rounds of rows) takes about 6
-// us however few there are; the per-row form 4.9 us at 128 tokens (here 6.3), 9.4
-// at 300 (here 6.8)
+// The prompt form from so many tokens and (token, head) rows on: a workgroup's chain
+// (factors, then four rounds of rows) takes 6.2 us at D = 128 and 4.3 at D = 64 however
+// few there are, the per-row form about 3.5 us and 0.3 per thousand rows.  us per row /
+// here: D = 128, 9216 rows (192 tokens of 48 heads) 5.9 / 6.3, 10752 (192 of 56) 6.7 /
+// 6.3, 2400 (300 of 8 + 1 heads) 4.0 / 6.3, 10000 (1000) 6.7 / 6.6; D = 64, 3456 rows 4.2 /
+// 4.3, 3072 4.0 / 4.35, 4320 4.5 / 4.3
 constexpr int kPromptMin = 192;
+constexpr int prompt_rows(int D) { return D == 128 ? 10240 : 4096; }
 
 constexpr int kPW = 8;        // waves of a workgroup
 
@@ -817,8 +821,8 @@ extern "C" int helm_qk_norm_rope_append(const void* qkv, const void* q_norm_w, c
   const int blocks = (items + 3) / 4;
   const PoolArgs pa = pool_args(pool);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // the prompt form from kPromptMin tokens on, where 16-byte accesses are aligned
-  if (B >= kPromptMin && helm::aligned16(qkv) && helm::aligned16(q_out) && helm::aligned16(q_norm_w) &&
+  // the prompt form from its line on, where 16-byte accesses are aligned
+  if (B >= kPromptMin && items >= prompt_rows(D) && helm::aligned16(qkv) && helm::aligned16(q_out) && helm::aligned16(q_norm_w) &&
       helm::aligned16(k_norm_w)) {
     const bool v_vec = helm::aligned16(pa.v) && pa.v_ss % 8 == 0 && pa.v_hs % 8 == 0 && pa.v_ds % 8 == 0;
     const dim3 grid((B + kTT - 1) / kTT, (Hq + Hkv + kHC - 1) / kHC + (Hkv + kHC - 1) / kHC);

@@ -673,11 +673,14 @@ def test_qk_norm_rope_cs_matches_transformers_ops(norm, shared_rows, rope_scalin
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,P,first,scatter", [(192, 32, 8, 128, 16, 0, False), (200, 40, 8, 128, 16, 5, False),
                                                         (233, 16, 8, 64, 32, 8, False), (199, 5, 1, 128, 64, 24, False),
-                                                        (250, 6, 3, 64, 16, 3, True), (305, 9, 9, 128, 8, 0, False)])
+                                                        (250, 6, 3, 64, 16, 3, True), (305, 9, 9, 128, 8, 0, False),
+                                                        (1463, 5, 1, 128, 64, 24, False), (343, 6, 3, 64, 16, 3, True),
+                                                        (385, 9, 9, 128, 8, 0, False), (214, 32, 8, 128, 16, 0, False)])
 def test_qk_norm_rope_append_prompt_form_equals_row_form(T, Hq, Hkv, D, P, first, scatter):
-    """helm_qk_norm_rope_append's prompt form (192 tokens on) writes the same bits as
-    its per-row form (the same tokens in calls of 48): a prompt from any offset of
-    its first page, tokens in scattered pages, rejected slots and offsets, head
+    """helm_qk_norm_rope_append writes the same bits for a prompt in one call (its prompt
+    form from 192 tokens and 10240 rows of 128 or 4096 of 64 on, which the last four
+    cases and the second and third reach) as for its tokens in calls of 48 (the per-row
+    form): a prompt from any offset of its first page, tokens in scattered pages, rejected slots and offsets, head
     counts that do not fill the eight of a workgroup."""
     from helm_amd.kernels import fused
     dev = torch.device("cuda")

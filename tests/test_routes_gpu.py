@@ -7,6 +7,7 @@ import torch
 from torch.profiler import ProfilerActivity, profile
 
 from helm_amd import kernels as hk
+from helm_amd.kernels import attention as ka
 from helm_amd.kernels import fused
 
 pytestmark = pytest.mark.gpu
@@ -119,3 +120,23 @@ def test_int8_form_by_size(M, N, K, kernel, tmp_path):
     mag = torch.mm(x.double().abs(), qs.abs()) * s.double()
     bound = mag * 2.0 ** -22 + exact.abs() * 2.0 ** -11 + 2.0 ** -24
     assert ((hk.int8_linear(x, q, s).double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("T,Hq,Hkv,D,prompt", [
+    (204, 32, 8, 128, False), (214, 32, 8, 128, True), (191, 64, 8, 128, False), (192, 64, 8, 128, True),
+    (1000, 8, 1, 128, False), (1024, 8, 1, 128, True), (300, 16, 8, 128, False),
+    (227, 14, 2, 64, False), (228, 14, 2, 64, True), (341, 8, 2, 64, False), (342, 8, 2, 64, True)])
+def test_kv_write_form_by_rows(T, Hq, Hkv, D, prompt, tmp_path):
+    """A prompt's q / k norm, RoPE and page write takes its prompt form from 192
+    tokens and 10240 (D = 64: 4096) rows on (the bits are the same in either)."""
+    dev = torch.device("cuda")
+    P, n = 16, -(-T // 16)
+    pool = ka.PoolView.of_pool(torch.zeros(n, Hkv, P, D, dtype=torch.float16, device=dev),
+                               ka.alloc_v((n, Hkv, P, D), torch.float16, dev, zero=True))
+    qkv = torch.randn(T, (Hq + 2 * Hkv) * D, device=dev).half()
+    w = torch.ones(D, dtype=torch.float16, device=dev)
+    pos = torch.arange(T, dtype=torch.int32, device=dev)
+    q = torch.empty(T, Hq, D, dtype=torch.float16, device=dev)
+    args = (qkv, w, w, 1e-6, pos, fused.rope_inv_freq(D, 1e6, dev), q, pool, pos // P, pos % P, Hq, Hkv, D, P)
+    (name, _), = launches(lambda: fused.qk_norm_rope_append(*args), tmp_path)
+    assert name.startswith("qk_norm_rope_append_prompt_kernel" if prompt else "qk_norm_rope_append_kernel"), name
