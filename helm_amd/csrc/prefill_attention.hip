@@ -13,9 +13,10 @@
 // consecutive keys whose V^T it feeds to the second MFMA.
 //
 // A workgroup is one kv head x a block of 4 * 16 * NC rows, one wave per 16 * NC
-// of them; rows are (query, head of the group) pairs, query-major, so a few
-// queries fill a block with all their heads (17 queries of a group of 4: one
-// block, not four) and a block spans fewer positions of the diagonal.  The four
+// of them; rows are (query, head of the group) pairs, query-major, so that few
+// queries over many keys fill a block with all their heads (17 queries of a group
+// of 4: one block, not four) and a block spans fewer positions of the diagonal; up
+// to kUnpackedMax queries in one pass they are the queries of one head.  The four
 // waves need the same K/V tiles, so the workgroup fetches each 32-key tile once,
 // straight into LDS (global_load_lds_dwordx4: every lane moves 16 bytes, a wave 1
 // KiB of contiguous pool memory), double buffered: tile s+1 is copied while tile s
@@ -89,7 +90,16 @@ struct PrefillArgs {
   int S;
   float* part_o;
   float* part_ml;
+  int pk, nsub;            // heads of a kv head's group packed into a block's rows (all, or 1 of nsub)
+  // 2^32 / d + 1 of the divisors pk, Hkv, nsub and S (mul_of), a division being some 30
+  // dependent instructions ahead of a block's first load
+  uint32_t mul_pk, mul_hkv, mul_sub;
 };
+
+// x / d as one high product: exact while x d < 2^32 (here x is below the rows of a
+// kv head, or the blocks of a launch; d below the heads).  d = 1 has no factor.
+__host__ inline uint32_t mul_of(int d) { return d > 1 ? (uint32_t)((1ull << 32) / (uint32_t)d + 1) : 0; }
+__device__ __forceinline__ int div_by(int x, uint32_t mul) { return mul ? (int)__umulhi((uint32_t)x, mul) : x; }
 
 // Workgroup barrier for the K/V stages: this wave's copies into LDS have landed
 // and its LDS reads have returned (s_waitcnt vmcnt(0) lgkmcnt(0); gfx9
@@ -161,23 +171,20 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   const int lane = tid & 63;
   const int col = lane & 15;
   const int grp = lane >> 4;
-  const int G = a.Hq / a.Hkv;
-  const int R = a.T * G;                           // rows (query, head of the group) of a kv head
+  const int G = a.pk;                              // heads that share a block
+  auto by_g = [&](int x) { return div_by(x, a.mul_pk); };
+  const int R = a.T * G;                           // rows (query, head) of those heads
   const int nqb = (R + kQB - 1) / kQB;
-  const int hk = (int)blockIdx.x % a.Hkv;
-  const int r = (int)blockIdx.x / a.Hkv;
-  const int sp = SPLIT ? r % a.S : 0;
-  const int q0 = (nqb - 1 - (SPLIT ? r / a.S : r)) * kQB;   // heaviest (latest) blocks first
+  const int r = div_by((int)blockIdx.x, a.mul_hkv);
+  const int hk = (int)blockIdx.x - r * a.Hkv;
+  const int rb = div_by(r, a.mul_sub);
+  const int sub = r - rb * (SPLIT ? a.S : a.nsub);
+  const int sp = SPLIT ? sub : 0;                  // key split, or
+  const int h0 = (SPLIT ? hk : hk * a.nsub + sub) * G;   // head subset of the kv head's group
+  const int q0 = (nqb - 1 - rb) * kQB;             // heaviest (latest) blocks first
   const int qw = q0 + wave * kWQ;                  // this wave's first row
-  int tq[NC], hq[NC];                              // query and head of this lane's columns
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int row = min(qw + c * 16 + col, R - 1);
-    tq[c] = row / G;
-    hq[c] = hk * G + (row - tq[c] * G);
-  }
 
-  const int wg_key_end = MASK ? a.kv_len : a.q_start + (min(q0 + kQB, R) - 1) / G + 1;
+  const int wg_key_end = MASK ? a.kv_len : a.q_start + by_g(min(q0 + kQB, R) - 1) + 1;
   const int npages = (wg_key_end + P - 1) / P;
   if (tid == 0) {
     s_bad = 0;
@@ -191,9 +198,13 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
     if (!ok) s_bad = 1;
   }
   // Q^T operands of the column tiles: lane holds q[query col][kk*32 + grp*8, +8]
+  int tq[NC], hq[NC];                              // query and head of this lane's columns
   h8_t qb_op[NC][KT];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
+    const int row = min(qw + c * 16 + col, R - 1);
+    tq[c] = by_g(row);
+    hq[c] = h0 + (row - tq[c] * G);
 #pragma unroll
     for (int kk = 0; kk < KT; ++kk)
       qb_op[c][kk] = ld_h8_nt(a.q + (int64_t)tq[c] * a.q_st + (int64_t)hq[c] * a.q_sh + kk * 32 + grp * 8);
@@ -203,7 +214,7 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   if constexpr (MASK) {
     if (a.key_end) {
       w_hi = 0;
-      for (int t = qw / G + lane; t <= (min(qw + kWQ, R) - 1) / G; t += 64) w_hi = max(w_hi, a.key_end[t]);
+      for (int t = by_g(qw) + lane; t <= by_g(min(qw + kWQ, R) - 1); t += 64) w_hi = max(w_hi, a.key_end[t]);
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) w_hi = max(w_hi, __shfl_xor(w_hi, off, 64));
       // wave-uniform after the butterfly: held in a scalar register
@@ -215,7 +226,7 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   __syncthreads();
 
   // keys [0, key_end) can be seen by some query of this wave
-  const int key_end = qw < R ? (MASK ? w_hi : a.q_start + (min(qw + kWQ, R) - 1) / G + 1) : 0;
+  const int key_end = qw < R ? (MASK ? w_hi : a.q_start + by_g(min(qw + kWQ, R) - 1) + 1) : 0;
   const int nsteps = (key_end + kKS - 1) / kKS;
   // the workgroup's steps [0, wg_steps): with MASK up to the last key any of its
   // rows sees (an LDS value, uniform over the workgroup).  Steps below a row's
@@ -225,7 +236,7 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
                             : (wg_key_end + kKS - 1) / kKS;
   // steps whose keys every query of the wave sees (all below the diagonal, valid
   // pages): no masking
-  const int nfull = (s_bad || MASK) ? 0 : min(nsteps, (a.q_start + qw / G + 1) / kKS);
+  const int nfull = (s_bad || MASK) ? 0 : min(nsteps, (a.q_start + by_g(qw) + 1) / kKS);
   const int p_last = max(npages - 1, 0);
   const uint16_t* kbase = a.k + (int64_t)hk * a.k_hs;
   const uint16_t* vbase = a.v + (int64_t)hk * a.v_hs;
@@ -498,6 +509,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a) {
       make_uint2(pack_h2(num[0] * inv, num[1] * inv), pack_h2(num[2] * inv, num[3] * inv));
 }
 
+// Up to this many queries a one-pass call keeps one head per block: its few steps
+// are chains of latencies, which a block of four busy waves lengthens (us packed /
+// one head: 32 heads of 128 at 32 queries 6.4 / 5.2, 64 7.1 / 6.1, 96 7.9 / 7.1, 128 8.5 /
+// 8.5; 28 heads over 4 at 17 6.4 / 5.0; with a mask 64 8.1 / 6.9).  Longer prompts gain
+// from packing (256 queries 11.3 / 11.4, 390 14.0 / 14.2, left-padded 1024 35.9 / 37.8).
+constexpr int kUnpackedMax = 96;
+
 // Key splits of a causal call.  A workgroup's steps are a serial chain of about a
 // microsecond each, so a grid that leaves workgroup slots empty is cut along the
 // keys, priced in steps: rounds of workgroups (two per CU) x the steps of a split
@@ -580,10 +598,15 @@ int prefill_launch(const char* fn, const void* q, int64_t q_stride_t, int64_t q_
   if (!ws || !helm::aligned16(ws) || ws_bytes < rows * (D + 2) * (int64_t)sizeof(float)) a.S = 1;
   a.part_o = static_cast<float*>(ws);
   a.part_ml = a.part_o ? a.part_o + rows * D : nullptr;
+  const int group = Hq / Hkv;
+  const bool packed = T > kUnpackedMax && (int64_t)T * group * group < (1ll << 32);   // div_by's range
+  a.pk = a.S > 1 || packed ? group : 1;
+  a.nsub = group / a.pk;
+  a.mul_pk = mul_of(a.pk); a.mul_hkv = mul_of(Hkv); a.mul_sub = mul_of(a.S > 1 ? a.S : a.nsub);
   auto go = [&](auto kern) {
     constexpr int qb = 64 * PF_NC;
-    const int nqb = (int)(((int64_t)T * (Hq / Hkv) + qb - 1) / qb);
-    hipLaunchKernelGGL(kern, dim3(nqb * Hkv * a.S), dim3(256), 0, s, a);
+    const int nqb = (int)(((int64_t)T * a.pk + qb - 1) / qb);
+    hipLaunchKernelGGL(kern, dim3(nqb * Hkv * a.nsub * a.S), dim3(256), 0, s, a);
   };
   auto by_page = [&](auto d_tag, auto m_tag, auto s_tag) {
     constexpr int Dc = decltype(d_tag)::value;

@@ -333,7 +333,11 @@ def test_fused_cs_attention_equals_norm_rope_append_attention(Hq, Hkv, D, P, seq
 @pytest.mark.parametrize("Hq,Hkv,D,P,T,q_start", [(32, 8, 128, 16, 300, 0), (40, 8, 128, 16, 257, 0),
                                                   (16, 8, 64, 32, 100, 0), (4, 1, 64, 64, 70, 0),
                                                   (32, 8, 128, 16, 77, 45), (8, 2, 128, 16, 1, 0),
-                                                  (8, 8, 64, 16, 33, 16), (16, 1, 128, 32, 200, 10)])
+                                                  (8, 8, 64, 16, 33, 16), (16, 1, 128, 32, 200, 10),
+                                                  # either side of the packed blocks' line
+                                                  (40, 8, 128, 16, 96, 0), (40, 8, 128, 16, 97, 0),
+                                                  (14, 2, 64, 16, 96, 40), (28, 4, 128, 64, 97, 30),
+                                                  (64, 8, 64, 32, 33, 0)])
 def test_prefill_attention_matches_causal_reference(Hq, Hkv, D, P, T, q_start):
     """helm_prefill_attn: query i (position q_start + i) over keys 0..q_start+i of
     scattered pages, against the fp64 causal form (bar 2e-3)."""
@@ -404,6 +408,23 @@ def test_prefill_attention_key_splits(Hq, Hkv, D, P, T, q_start):
     assert np.array_equal(outs[0], outs[2])
 
 
+def test_prefill_attention_more_heads_than_a_packed_block_divides():
+    """2048 query heads over one kv head: (query, head) rows past the range in which
+    the kernel's row / heads is exact keep one head per block."""
+    g = torch.Generator(device="cuda").manual_seed(5)
+    T, Hq, D, P = 1024, 2048, 64, 16
+    k = torch.randn(T // P, 1, P, D, generator=g, device="cuda").half()
+    v = ka.alloc_v((T // P, 1, P, D), device="cuda")
+    v.copy_(torch.randn(T // P, 1, P, D, generator=g, device="cuda"))
+    q = torch.randn(T, Hq, D, generator=g, device="cuda").half()
+    out = ka.prefill_attention(q, ka.PoolView.of_pool(k, v),
+                               torch.arange(T // P, dtype=torch.int32, device="cuda"), P)
+    kd, vd = (t.reshape(T, D).double().contiguous() for t in (k, v.contiguous()))
+    for t in (0, 127, 128, 517, T - 1):
+        p = torch.softmax(torch.mm(q[t].double(), kd[:t + 1].t().contiguous()) / math.sqrt(D), -1)
+        assert (out[t].double() - torch.mm(p, vd[:t + 1])).abs().max() <= ATOL
+
+
 def _mask_case(kind, Hq, T, N, g):
     """Masks of the shapes a drop-in prefill receives: [Hm, T, N]."""
     causal = np.arange(N)[None, :] <= np.arange(T)[:, None] + (N - T)
@@ -430,7 +451,11 @@ def _mask_case(kind, Hq, T, N, g):
                                                  (4, 1, 64, 64, 70, 70, "full"),
                                                  (8, 2, 128, 16, 1, 45, "per_head"),
                                                  (32, 8, 128, 16, 129, 2049, "hf_min"),
-                                                 (40, 8, 128, 16, 700, 700, "left_pad")])
+                                                 (40, 8, 128, 16, 700, 700, "left_pad"),
+                                                 (40, 8, 128, 16, 96, 96, "left_pad"),
+                                                 (28, 4, 128, 64, 97, 97, "hf_min"),
+                                                 (14, 2, 64, 16, 64, 100, "per_head"),
+                                                 (40, 8, 128, 16, 97, 130, "per_head")])
 @pytest.mark.parametrize("key_ranges", [True, False])
 def test_prefill_attention_mask_matches_reference(Hq, Hkv, D, P, T, N, kind, key_ranges):
     """helm_prefill_attn_mask: T queries over N keys of scattered pages with an

@@ -140,3 +140,22 @@ def test_kv_write_form_by_rows(T, Hq, Hkv, D, prompt, tmp_path):
     args = (qkv, w, w, 1e-6, pos, fused.rope_inv_freq(D, 1e6, dev), q, pool, pos // P, pos % P, Hq, Hkv, D, P)
     (name, _), = launches(lambda: fused.qk_norm_rope_append(*args), tmp_path)
     assert name.startswith("qk_norm_rope_append_prompt_kernel" if prompt else "qk_norm_rope_append_kernel"), name
+
+
+@pytest.mark.parametrize("T,past,Hq,Hkv,D,workgroups", [
+    (96, 0, 40, 8, 128, 40), (97, 0, 40, 8, 128, 8 * 4), (17, 0, 28, 4, 64, 28), (1, 0, 8, 1, 128, 8),
+    (130, 0, 8, 8, 64, 16)])
+@pytest.mark.parametrize("masked", [False, True])
+def test_prefill_blocks_by_queries(T, past, Hq, Hkv, D, workgroups, masked, tmp_path):
+    """One pass over few queries keeps one head per 128-row block (up to 96 of them),
+    longer prompts pack the heads of a group."""
+    dev = torch.device("cuda")
+    P, n = 16, -(-(past + T) // 16)
+    pool = ka.PoolView.of_pool(torch.zeros(n, Hkv, P, D, dtype=torch.float16, device=dev),
+                               ka.alloc_v((n, Hkv, P, D), torch.float16, dev, zero=True))
+    q = torch.randn(T, Hq, D, device=dev).half()
+    table = torch.arange(n, dtype=torch.int32, device=dev)
+    mask = torch.ones(1, T, T, dtype=torch.bool, device=dev) if masked else None
+    seen = launches(lambda: ka.prefill_attention(q, pool, table, P, past, mask=mask), tmp_path)
+    attn = [n for name, n in seen if name.startswith("prefill_attn_kernel")]
+    assert attn == [workgroups], seen
