@@ -85,17 +85,23 @@ def choose_num_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: 
 def choose_batch_splits(batch: int, num_kv_heads: int, max_pages: int, page_size: int = 16) -> int:
     """Split count of one attention call over `batch` items whose lengths the host
     does not know: with choose_num_splits the workgroups of the longest item are the
-    whole launch's tail while the short items' ones have ended.  From four items on
-    the count is doubled, from eight tripled (the CUs then take the longest item's
-    extra workgroups as the short ones end), to splits of at least 256 tokens.
-    Measured against choose_num_splits with lengths spread over 1/16 .. 1 of the
-    longest: 8 items of 12000 tokens 50.0 -> 33.9 us, 16 of 8000 65.0 -> 43.9, 4 of 4000
-    13.2 -> 11.6; the price where all are equal (more partials to merge): 63.9 -> 65.6,
-    83.8 -> 85.8, 15.0 -> 15.3.  Two or three items stay (two equal ones of 16384 25.3 ->
-    26.1 us), and four times as many splits cost equal lengths up to 15%."""
+    whole launch's tail while the short items' ones have ended.  From eight items on
+    the count is tripled where that leaves a split 960 tokens, from four doubled where
+    it leaves 240 (the CUs then take the longest item's extra workgroups as the short
+    ones end).  Only whole multiples: workgroups that fill no whole number of rounds
+    cost equal lengths up to 19% (7 splits instead of 5 for 6 items of 2000 tokens 13.5 ->
+    15.9 us; 46 instead of 32 for 4 of 12000 with 2 kv heads 9.4 -> 11.2).
+    Measured over 4-16 items of 1000-12000 tokens in six head shapes, against
+    choose_num_splits: lengths spread over 1/16 .. 1 of the longest 16% less time in the
+    mean (8 items of 12000 tokens 51.1 -> 32.4 us, 16 of 8192 67.9 -> 39.9, 4 of 4000 13.6 ->
+    12.0) and nowhere more; equal lengths 0.3% more in the mean and at most 6% (more
+    partials to merge: 64.4 -> 65.6, 89.9 -> 86.8, 15.6 -> 15.5).  Two or three items stay
+    (two equal ones of 16384 25.3 -> 26.1 us)."""
     base = choose_num_splits(batch, num_kv_heads, max_pages, page_size)
-    more = 1 if batch < 4 else 2 if batch < 8 else 3
-    return max(base, min(more * base, max_pages * page_size // 256))
+    tokens = max_pages * page_size
+    if batch >= 8 and tokens // (3 * base) >= 960:
+        return 3 * base
+    return 2 * base if batch >= 4 and tokens // (2 * base) >= 240 else base
 
 
 def alloc_v(shape, dtype=torch.float16, device=None, pin_memory: bool = False,

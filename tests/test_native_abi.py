@@ -206,6 +206,24 @@ def test_split_count_rule(batch, P):
     assert choose_num_splits(1, 8, 1042, 16) == 32 and split_pages(1042, 32, 16) == 34
 
 
+@pytest.mark.parametrize("P", [16, 64])
+@pytest.mark.parametrize("hkv", [1, 2, 4, 8, 32])
+def test_batch_splits_are_whole_multiples(hkv, P):
+    """choose_batch_splits: once, twice (from four items) or three times (from eight)
+    choose_num_splits and nothing between, as workgroups that fill part of a round
+    slow equal lengths down; a larger count leaves each split 240 / 960 tokens."""
+    from helm_amd.kernels.attention import choose_batch_splits, choose_num_splits
+    for batch in (1, 2, 3, 4, 5, 6, 7, 8, 12, 16, 40):
+        for tokens in (16, 200, 1000, 2000, 4000, 8192, 12000, 32768):
+            n = -(-tokens // P)
+            base, got = choose_num_splits(batch, hkv, n, P), choose_batch_splits(batch, hkv, n, P)
+            times = got // base
+            assert got == times * base and times in ((1,) if batch < 4 else (1, 2) if batch < 8 else (1, 2, 3))
+            assert times == 1 or n * P >= got * (240 if times == 2 else 960)
+    assert choose_batch_splits(4, 2, 750, 16) == 32 and choose_batch_splits(6, 8, 125, 16) == 5
+    assert choose_batch_splits(8, 8, 750, 16) == 12
+
+
 def test_kv_append_rejects_small_pool_strides():
     fake = ctypes.c_void_p(16)
     from helm_amd.kernels.attention import KvPoolStruct
