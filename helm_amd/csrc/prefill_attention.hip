@@ -520,8 +520,10 @@ constexpr int kUnpackedMax = 96;
 // microsecond each, so a grid that leaves workgroup slots empty is cut along the
 // keys, priced in steps: rounds of workgroups (two per CU) x the steps of a split
 // and its start, plus the partials' traffic and the merge launch.  From 129
-// workgroups on, up to 2048 keys stay one pass: little to gain, and a row's bits
-// then do not depend on how its prompt was chunked.
+// workgroups on, up to 2048 keys stay one pass: little to gain, and between chunks
+// of that size a row's bits do not depend on where a prompt was cut.  Smaller chunks
+// are split whatever their length (390 queries after 390 of 32 heads: two splits),
+// and a split's probabilities are rounded to fp16 relative to its own maximum.
 int prefill_splits(int T, int q_start, int Hq, int Hkv, int D) {
   const int64_t keys = (int64_t)q_start + T;
   const int64_t blocks = ((int64_t)T * (Hq / Hkv) + 64 * PF_NC - 1) / (64 * PF_NC) * Hkv;

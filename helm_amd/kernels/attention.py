@@ -439,6 +439,8 @@ def prefill_attention(q: torch.Tensor, pool: PoolView, page_table: torch.Tensor,
     """Causal attention of the T queries q [T, Hq, D] (positions q_start ..
     q_start+T-1) over the keys 0 .. q_start+T-1 of one sequence's pages
     (page_table [>= ceil((q_start+T)/P)] int32 slots).  Returns [T, Hq, D] fp16.
+    A call of few queries over many keys splits the keys, so a prompt's rows can differ
+    in their last bits with the chunks (T, q_start) it is attended in.
 
     With `mask` ([Hm, T, kv_len], Hm 1 or Hq, bool or additive; q_start must be 0)
     every query sees keys 0 .. kv_len-1 instead, with the mask added to its scaled

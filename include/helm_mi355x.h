@@ -250,8 +250,11 @@ int helm_prefill_attn(const void* q, int64_t q_stride_t, int64_t q_stride_h,
  * helm_prefill_attn_workspace_bytes (16-byte aligned; its contents on entry do not
  * matter): calls whose rows leave workgroup slots empty (few queries over many
  * cached keys) then also split the keys, keep fp32 partials there and merge them in
- * a second kernel.  Same results up to the fp32 summation order; without the
- * workspace (null, or too small) as helm_prefill_attn. */
+ * a second kernel.  Same results up to the fp32 summation order and to the fp16
+ * rounding of the probabilities, which is relative to a split's own maximum; without
+ * the workspace (null, or too small) as helm_prefill_attn.  Whether a call is split
+ * depends on its T and q_start, so the bits of a prompt's rows can depend on the chunks
+ * it is attended in; helm_prefill_attn splits no call. */
 int64_t helm_prefill_attn_workspace_bytes(int T, int q_start, int Hq, int Hkv, int D);
 int helm_prefill_attn_ws(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                          const helm_kv_pool* pool, const int32_t* page_table,

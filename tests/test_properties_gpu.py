@@ -26,6 +26,7 @@ import math
 import pytest
 import torch
 
+from helm_amd import _native
 from helm_amd.kernels import attention as ka
 from helm_amd.kernels import fused
 
@@ -234,7 +235,8 @@ def test_prefill_attention_pages_and_chunks(Hq_):
     layouts): moving every page to another slot gives the same bits, and a prompt
     attended in two chunks (queries 0..c-1, then c..2047 with q_start = c, at a
     split that is a multiple of the 32-row wave tile and at one that is not) gives
-    the same rows as one call: key steps a query cannot see add exactly nothing."""
+    the same rows as one call: key steps a query cannot see add exactly nothing.
+    (Chunks whose keys are split: test_prefill_attention_short_chunks.)"""
     T = 2048
     npg = T // P
     g = torch.Generator(device=DEV).manual_seed(Hq_)
@@ -260,3 +262,38 @@ def test_prefill_attention_pages_and_chunks(Hq_):
     assert torch.equal(out_moved, out)
     for c, o in chunks.items():
         assert torch.equal(o, out), f"chunked at {c}"
+
+
+@pytest.mark.parametrize("Hq_", [40, 32])
+@pytest.mark.parametrize("cut", [96, 97, 1700, 1985, 2040])
+def test_prefill_attention_short_chunks(Hq_, cut):
+    """A chunk of few queries (128 workgroups or fewer) has its keys split: its rows
+    equal the one call's up to the fp16 rounding of the probabilities, which is
+    relative to a split's own maximum (2^-11 of each weighted value in either call),
+    and the two final roundings; a repeated call gives the same bits.  Without the
+    workspace nothing is split and the bits are the one call's for every cut."""
+    T = 2048
+    g = torch.Generator(device=DEV).manual_seed(Hq_ + cut)
+    k = torch.randn(T // P, Hkv, P, D, device=DEV, generator=g).half()
+    v = torch.randn(T // P, Hkv, P, D, device=DEV, generator=g).half()
+    pt = torch.randperm(T // P, device=DEV, generator=g).int()
+    q = torch.randn(T, Hq_, D, device=DEV, generator=g).half()
+    pool, scale = _pool(k, v), 1.0 / math.sqrt(D)
+    out = ka.prefill_attention(q, pool, pt, P, 0, scale)
+
+    def one_pass(a, b):
+        o = torch.empty(b - a, Hq_, D, dtype=torch.float16, device=DEV)
+        _native.call("helm_prefill_attn", q[a:b].data_ptr(), q.stride(0), q.stride(1), pool.c_ref(),
+                     pt.data_ptr(), a, b - a, Hq_, Hkv, D, P, scale, o.data_ptr(), o.stride(0),
+                     o.stride(1), torch.cuda.current_stream().cuda_stream)
+        return o
+
+    assert torch.equal(torch.cat([one_pass(0, cut), one_pass(cut, T)]), out)
+    split = False
+    for a, b in ((0, cut), (cut, T)):
+        o = ka.prefill_attention(q[a:b], pool, pt, P, a, scale)
+        assert torch.equal(ka.prefill_attention(q[a:b], pool, pt, P, a, scale), o)
+        split |= _native.lib().helm_prefill_attn_workspace_bytes(b - a, a, Hq_, Hkv, D) > 0
+        bound = 2.0 ** -10 * (v.float().abs().max() + out[a:b].float().abs())
+        assert ((o.float() - out[a:b].float()).abs() <= bound).all()
+    assert split == (cut > 1024)

@@ -119,7 +119,9 @@ def test_int8_form_by_size(M, N, K, kernel, tmp_path):
     exact = torch.mm(x.double(), qs) * s.double()
     mag = torch.mm(x.double().abs(), qs.abs()) * s.double()
     bound = mag * 2.0 ** -22 + exact.abs() * 2.0 ** -11 + 2.0 ** -24
-    assert ((hk.int8_linear(x, q, s).double() - exact).abs() <= bound).all()
+    y = hk.int8_linear(x, q, s)
+    assert ((y.double() - exact).abs() <= bound).all()
+    assert torch.equal(hk.int8_linear(x, q, s), y)
 
 
 @pytest.mark.parametrize("T,Hq,Hkv,D,prompt", [
