@@ -304,9 +304,10 @@ def test_int8_linear_module_and_patch():
                                    (3, 4113, 4096)])
 def test_fused_norm_residual_and_swiglu(M, N, K):
     """RMSNorm prologue + residual / SwiGLU epilogues: the streaming kernel at 1-2
-    tokens and where K is not 4096 (two rows per wave at 3-4 tokens; ragged N
+    tokens and at 3-4 beyond K = 6144 (two rows per wave at 3-4 tokens; ragged N
     leaves a wave's second row past the end), the matrix-core forms with the
-    norm applied to their x copy in LDS at 3-16 tokens and K = 4096."""
+    norm applied to their x copy in LDS at 3-16 tokens and K = 4096, to x^T in
+    registers at other K (5120 here; test_x_in_registers_int8_norm)."""
     g = np.random.default_rng(21 + M)
     x = g.standard_normal((M, K)).astype(np.float16)
     nw = (1.0 + 0.1 * g.standard_normal(K)).astype(np.float16)
@@ -411,15 +412,18 @@ def test_small_m_residual_and_bias(M):
 
 @pytest.mark.parametrize("M,N,K", [(7, 4096, 12288), (8, 4096, 12288), (12, 4096, 12288),
                                    (16, 4096, 12288), (16, 1000, 6144), (9, 68, 24576),
-                                   (16, 4098, 9216)])
+                                   (16, 4098, 9216), (8, 4096, 9216), (16, 3844, 12288),
+                                   (12, 3076, 15360), (9, 2000, 24576), (14, 8132, 6144)])
 def test_small_m_split_k_workspace(M, N, K):
     """Long K at 8-16 tokens through helm_int8_gemv_ws: k split over workgroups
-    (3072 each), fp32 partial sums in the caller's workspace, then one reduce with
+    (3072 each, or x^T in registers by its own slices: 16 x 1000 x 6144 and 9 x 68 x
+    24576), fp32 partial sums in the caller's workspace, then one reduce with
     scale, bias and the residual aliasing y.  The workspace is filled with NaN
-    first (its contents on entry must not matter); 64-row groups past N (N = 1000,
-    68), a grid below the CU count (N = 68), and 7 tokens or N % 4 != 0 (no
-    workspace, one-pass forms) are covered.  Checked against the fp64 closed form and against the
-    one-pass form without a workspace (fp32 summation order only)."""
+    first (its contents on entry must not matter); 64-row groups past N (N = 3844,
+    3076, 2000, 8132), a grid below the CU count (9216 -> 4096: 192), and 7 tokens or
+    N % 4 != 0 (no workspace, one-pass forms) are covered.  Checked against the fp64
+    closed form and against the one-pass form without a workspace (fp32 summation
+    order only)."""
     from helm_amd import _native
     g = np.random.default_rng(K + N + M)
     x, q, s, b = make_inputs(M, N, K, seed=K + 7 * N + M, bias=True)
@@ -618,6 +622,68 @@ def test_x_in_registers_fp16(M, N, K):
     wk[N // 2] = 0
     bound = (x.double().cpu().abs() @ wk.t()) * 2.0 ** -22 + exact.nan_to_num(0, 0, 0).abs() * 2.0 ** -11 + 2.0 ** -24
     assert ((y - exact).abs() <= bound)[:, keep].all()
+
+
+def rms_normed(x, w, eps):
+    """fp16(w * fp16(x * rsqrt(mean(x^2) + eps))), as Qwen3RMSNorm rounds for fp16."""
+    x32 = x.astype(np.float32)
+    rstd = 1.0 / np.sqrt((x32 ** 2).mean(-1, keepdims=True) + eps)
+    return (w.astype(np.float32) * (x32 * rstd).astype(np.float16).astype(np.float32)).astype(np.float16)
+
+
+def norm_flip_bound(xn, wmax):
+    """What a few normalised elements on their neighbouring fp16 value change in an
+    output: the fp32 sum of squares in another order moves rsqrt by some 2^-23, which
+    puts about one element in 4000 (2^-23 against a spacing of 2^-11 .. 2^-10) across a
+    rounding edge; eight of K <= 6144, each 2^-10 of itself and at most the largest, times
+    the weight."""
+    return 8 * 2.0 ** -10 * np.abs(xn.astype(np.float64)).max(-1, keepdims=True) * wmax
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 17, 16), (5, 200, 144), (16, 1001, 1024), (9, 333, 1040), (12, 4099, 2560),
+                                   (7, 48, 5104), (16, 515, 5120), (13, 4113, 5120), (4, 31, 6128), (16, 100, 6144)])
+def test_x_in_registers_int8_norm(M, N, K):
+    """The RMSNorm prologue of the kernel with x^T in registers at 3-16 tokens: K that
+    ends inside a unit or leaves waves none, one to six units a wave, several row
+    tiles, a token of zeros; with a bias, with a residual aliasing y, and in the
+    SwiGLU launch."""
+    g = np.random.default_rng(3 * K + N + M)
+    x, q, s, b = make_inputs(M, N, K, seed=K + N + M, bias=True)
+    _, q2, s2, _ = make_inputs(M, N, K, seed=K + 5 * N + M)
+    x[M // 2] = 0
+    nw = (1.0 + 0.1 * g.standard_normal(K)).astype(np.float16)
+    res = g.standard_normal((M, N)).astype(np.float16)
+    xd, nwd, qd, sd, bd, resd, q2d, s2d = to_dev(x, nw, q, s, b, res, q2, s2)
+    xn = rms_normed(x, nw, 1e-5)
+    lin = ol.int8_linear_exact(xn, q, s, b)
+    bound = accumulation_bound(xn, q, s) + norm_flip_bound(xn, 127 * s.astype(np.float64)[None, :])
+    y = fused.int8_gemv_fused(xd, qd, sd, norm_weight=nwd, eps=1e-5, bias=bd).cpu().numpy()
+    assert_linear_ok(y, lin, f"norm M={M} N={N} K={K}", bound)
+    y = resd.clone()
+    fused.int8_gemv_fused(xd, qd, sd, norm_weight=nwd, eps=1e-5, bias=bd, residual=y, out=y)
+    exp = res.astype(np.float64) + lin.astype(np.float16).astype(np.float64)
+    assert (np.abs(y.cpu().numpy().astype(np.float64) - exp) <= ulp16(lin) + bound + ulp16(exp)).all()
+    a = fused.int8_gemv_swiglu(xd, qd, sd, q2d, s2d, norm_weight=nwd, eps=1e-5).cpu().numpy()
+    gt, up = (ol.int8_linear_exact(xn, *w).astype(np.float16).astype(np.float64) for w in ((q, s), (q2, s2)))
+    assert swiglu_within_bar(a, gt, up)
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 1000, 960), (16, 77, 1088), (8, 300, 2112), (12, 515, 2560), (9, 2000, 3584),
+                                   (16, 130, 4160), (5, 33, 4992), (4, 16, 5120), (3, 4200, 3008)])
+def test_x_in_registers_fp16_norm(M, N, K):
+    """fp16 weights with the norm prologue and x^T in registers: 2, 4, 8 and 10 units a
+    wave, K that does not fill them, ragged N, a token of zeros."""
+    g = np.random.default_rng(K + N + M)
+    x = g.standard_normal((M, K)).astype(np.float16)
+    x[M - 1] = 0
+    nw = (1.0 + 0.1 * g.standard_normal(K)).astype(np.float16)
+    w = (g.standard_normal((N, K)) * 0.05).astype(np.float16)
+    xd, nwd, wd = to_dev(x, nw, w)
+    y = fused.fp16_gemv_rmsnorm(xd, nwd, 1e-5, wd).cpu().numpy().astype(np.float64)
+    xn, w64 = rms_normed(x, nw, 1e-5).astype(np.float64), w.astype(np.float64)
+    exact = xn @ w64.T
+    bound = np.abs(xn) @ np.abs(w64).T * 2.0 ** -22 + norm_flip_bound(xn, np.abs(w64).max(-1)[None, :])
+    assert (np.abs(y - exact) <= ulp16(exact) + bound).all()
 
 
 @pytest.mark.parametrize("M,N,K", [(17, 64, 64), (32, 1001, 256), (33, 4099, 1024), (64, 130, 4160), (77, 12288, 1088),
