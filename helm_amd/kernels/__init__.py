@@ -73,8 +73,10 @@ def dequantize(qweight: torch.Tensor, scale: torch.Tensor) -> torch.Tensor:
 def _flatten(x: torch.Tensor, K: int, what: str) -> torch.Tensor:
     if x.shape[-1] != K:
         raise RuntimeError(f"{what}: input last dim ({x.shape[-1]}) != weight K ({K})")
+    if x.dim() == 2 and x.stride() == (K, 1) and K % 8 == 0 and x.data_ptr() % 16 == 0:
+        return x
     # (reshape states the stride of a single row as K, whatever the view's says)
-    x2 = x if x.dim() == 2 and x.stride(0) == K else x.reshape(-1, K)
+    x2 = x.reshape(-1, K)
     if x2.stride(-1) != 1 or x2.stride(0) % 8 != 0 or x2.data_ptr() % 16 != 0:
         x2 = x2.contiguous()
     return x2
@@ -102,7 +104,9 @@ def int8_linear(input: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
     M = x2.shape[0]
     if out is None:
         out = torch.empty((*input.shape[:-1], N), dtype=torch.float16, device=input.device)
-    y2 = out if out.dim() == 2 and out.shape[1] == N and out.stride(0) == N else out.view(-1, N)
+        y2 = out if input.dim() == 2 else out.view(-1, N)
+    else:
+        y2 = out.view(-1, N)
     if M == 0:
         return out
     stream = _native.stream_ptr(input.device)
