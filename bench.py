@@ -338,7 +338,7 @@ def sweep_gemv() -> None:
         for M in (1, 4, 16):
             x = torch.randn(M, K, device=dev, generator=g).half()
             y = torch.empty(M, N, device=dev).half()
-            wsb = int(_native.lib().helm_int8_gemv_workspace_bytes(M, N, K))
+            wsb = int(_native.lib().helm_int8_gemv_split_bytes(M, N, K))
             ws = torch.empty(max(wsb, 16), dtype=torch.uint8, device=dev)
 
             def fn(i):

@@ -383,9 +383,10 @@ int pick_tn(int M, int N) {
 // 12288), so what counts is how many chains run at once and how long each is.  Here
 // tiles are 64 columns wide and as tall as the rows need (32 RT), two to four
 // workgroups fit a CU, and K is split over workgroups until they fill, partial sums
-// in fp32.  Against the prompt form alone, us: 77 tokens 17408 -> 5120 126 -> 43, 4096
-// -> 4096 32.4 -> 16.8, 4096 -> 1024 32.2 -> 12.0, 4096 -> 12288 33.5 -> 29.9; 17 tokens
-// 4096 -> 12288 33.4 -> 19.9; 256 tokens 17408 -> 5120 127 -> 78.
+// in fp32.  Against the prompt form alone, us, weights rotating through HBM: 77 tokens
+// 17408 -> 5120 126 -> 40, 4096 -> 4096 32.6 -> 16.5, 4096 -> 1024 32.3 -> 12.2, 4096 -> 12288
+// 33.3 -> 28.9 (32.5 -> 24.6 with the matrix in the last-level cache); 17 tokens 4096 -> 12288
+// 33.3 -> 19.3; 256 tokens 17408 -> 5120 126 -> 70.
 struct Skinny {
   int rt, s;        // row tiles per wave (0: not this form), k slices
 };

@@ -1,6 +1,6 @@
 // gemv_small_m.hip — INT8 weight-only linear for 3 <= M <= 16 tokens.
 //
-// Reached for K = 4096, for long K whose 16-row tiles fill the CUs in one round, for
+// Reached for K = 4096, for other K whose grid here is whole rounds of the CUs, for
 // calls without the workspace that gemv_xreg.hip needs for long K, and (fp16 weights)
 // for K below 2048 or beyond 5120 and for many outputs at K whose units
 // gemv_xreg.hip does not walk whole; gemv_xreg.hip takes the rest.

@@ -25,9 +25,9 @@
 // Longer K (int8 only): workgroup b takes k slice b % S of S, fp32 partial sums
 // go to the caller's workspace and a second kernel adds them and applies the
 // epilogue.
-// Measured: 5120 -> 2 x 17408 with norm and SwiGLU at 12 tokens 345 -> 37.8 us (4.7
-// TB/s), 17408 -> 5120 at 8 tokens 34.4 -> 23.9 us, fp16 4096 -> 151936 at 4 tokens
-// 233 -> 194 us (6.4 TB/s).  Between two sizes of one shape the rate is 6.9 TB/s;
+// Measured, weights rotating through HBM: 5120 -> 2 x 17408 with norm and SwiGLU at 12
+// tokens 344 -> 36.5 us (4.9 TB/s), 17408 -> 5120 at 8 tokens 32.8 -> 22.9 us, fp16 4096 ->
+// 151936 at 4 tokens 221 -> 189 us (6.6 TB/s).  Between two sizes of one shape the rate is 6.9 TB/s;
 // 5-9 us of a launch are its start (x from L2: 160 KB per CU at 16 tokens) and end.
 #include <algorithm>
 #include <type_traits>

@@ -27,10 +27,11 @@
 //
 // A step is a serial chain of about 2000 cycles (operand reads, QK, softmax, PV); per
 // step 64 KB of LDS reads a workgroup, 512 cycles of MFMA a wave and about as many
-// of VALU work bound it, two workgroups per CU overlap.  Measured: 14B heads at T =
-// 2048 74.5 -> 67.1 us (641 TFLOP/s), 390 queries of 32 heads over 7000 cached keys
-// (104 workgroups, four key splits) 198 -> 84 us, T = 4096 over 12000 keys 1305 -> 1221
-// us (966 TFLOP/s), left-padding mask at T = 2048 171 -> 151 us.
+// of VALU work bound it, two workgroups per CU overlap.  Measured before packing,
+// early copies and key splits -> now, graph replays over the same inputs (K/V in the
+// last-level cache): 40 heads at T = 2048 65.7 -> 60.0 us (716 TFLOP/s), 4096 204 -> 192,
+// 390 queries of 32 heads over 7000 cached keys (104 workgroups, four key splits) 195 ->
+// 73.5, a left-padding mask over a fifth at T = 2048 98 -> 77 (the kernel alone).
 //
 // LDS layouts (16-byte chunks) are chosen so that both the copies and the operand
 // reads are conflict free:
@@ -230,8 +231,8 @@ __global__ __launch_bounds__(256, PF_WPE) void prefill_attn_kernel(PrefillArgs a
   const int nsteps = (key_end + kKS - 1) / kKS;
   // the workgroup's steps [0, wg_steps): with MASK up to the last key any of its
   // rows sees (an LDS value, uniform over the workgroup).  Steps below a row's
-  // first visible key are visited anyway (their keys are -inf for it): a loop
-  // starting at a run-time step measured spills at every form tried.
+  // first visible key are visited anyway (their keys are -inf for it); only the
+  // SPLIT form starts at a step of its own.
   const int wg_steps = MASK ? (__builtin_amdgcn_readfirstlane(s_kr) + kKS - 1) / kKS
                             : (wg_key_end + kKS - 1) / kKS;
   // steps whose keys every query of the wave sees (all below the diagonal, valid

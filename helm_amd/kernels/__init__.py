@@ -19,7 +19,7 @@ load_error() :97-100                   load_error()
 
 Dispatch follows the reference's shape rule (fp16_linear :72-88): a call whose
 leading dims multiply to <= 16 tokens is a decode GEMV (helm_int8_gemv_ws /
-helm_fp16_gemv), a larger one a prefill GEMM (helm_int8_gemm on MFMA).  Unlike the
+helm_fp16_gemv), a larger one a prefill GEMM (helm_int8_gemm_ws on MFMA).  Unlike the
 reference there is no fallback: a missing library or a CPU tensor raises
 RuntimeError.
 """

@@ -80,7 +80,7 @@ def int8_gemv_fused(x: torch.Tensor, qweight: torch.Tensor, scale: torch.Tensor,
             y2.copy_(r2)
             res = y2.data_ptr()
     if norm_weight is None:
-        # no norm prologue: the workspace form (split K for long K at 5-16 tokens)
+        # no norm prologue: the workspace form (split K for long K at 3-16 tokens)
         ws_bytes = gemv_split_bytes(M, N, K)
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
         _native.call("helm_int8_gemv_ws", x2.data_ptr(), x2.stride(0), qweight.data_ptr(),

@@ -47,9 +47,9 @@ from .kv_allocator import KVAllocator
 from .kv_cache import KVCacheManager
 from .page_table import DevicePageTable, PinnedRing
 
-# hidden size whose RMSNorms run inside the matrix-core GEMVs at 3-16 items
-# (helm_int8_gemv_fused / helm_int8_gemv_swiglu with a norm weight take K = 4096
-# there).  Every workgroup normalises its own x copy, which pays for the
+# hidden size whose RMSNorms run inside the matrix-core GEMVs at 3-16 items (the
+# norm-fused calls take every K up to 6144 there, but the step has been compared at
+# 4096 only: other hidden sizes keep a separate RMSNorm).  Every workgroup normalises its own x copy, which pays for the
 # gate / up + SwiGLU launch at every item count (4096 -> 2 x 12288: 8 items 20.2
 # against 21.4 us with a separate RMSNorm) but for q|k|v only up to 4 items (8.8
 # against 10.3 us; 16 items 18.3 against 14.2 us).

@@ -75,9 +75,9 @@ int helm_fp16_gemv(const void* x, int64_t ldx, const void* w, int64_t ldw,
  * helm/runtime/kv_offload.py:241-271 and transformers' Qwen3DecoderLayer).
  *   norm_w != NULL: x is first RMS-normalised per token,
  *       xn = fp16( norm_w * fp16( x * rsqrt(mean(x^2) + eps) ) )
- *       (at 3-16 tokens and K = 4096 inside the matrix-core kernel, each
- *       workgroup normalising its own copy: from 5 tokens on, helm_rmsnorm and
- *       the call without norm_w are faster for the plain linear)
+ *       (at 3-16 tokens and K up to 6144 inside the matrix-core kernels, each
+ *       workgroup normalising its own copy: at K = 4096 from 5 tokens on, helm_rmsnorm
+ *       and the call without norm_w are faster for the plain linear)
  *   residual != NULL: y = fp16( residual + fp16(linear(x)) ), residual [M, N] row
  *       stride ldy (may alias y). */
 int helm_int8_gemv_fused(const void* x, int64_t ldx, const void* norm_w, float eps,
@@ -87,13 +87,12 @@ int helm_int8_gemv_fused(const void* x, int64_t ldx, const void* norm_w, float e
 
 /* helm_int8_gemv_fused without the norm prologue, with a caller-owned workspace
  * of helm_int8_gemv_workspace_bytes(M, N, K) bytes (16-byte aligned; its contents
- * on entry do not matter).  Shapes whose activations of 8-16 tokens exceed the
- * kernel's LDS (K a multiple of 3072 above 4096, N % 4 == 0, e.g. the Qwen3-8B
- * down projection 12288 -> 4096) then split K over workgroups, keep fp32 partial
- * sums there and reduce them in a second kernel; every other shape may pass
- * workspace NULL and then runs as helm_int8_gemv_fused, or
- * helm_int8_gemv_split_bytes of workspace for the split form of other long K.  Same results
- * up to the fp32 summation order.  Replaces the same decode fast path as
+ * on entry do not matter).  That is 0 except at 8-16 tokens for K a multiple of 3072
+ * above 4096 and N % 4 == 0 (e.g. the Qwen3-8B down projection 12288 -> 4096), which
+ * require it; every other shape may pass workspace NULL and then runs as
+ * helm_int8_gemv_fused, or helm_int8_gemv_split_bytes of workspace.  With it, long K
+ * is split over workgroups where that is the faster form: fp32 partial sums there,
+ * added by a second kernel.  Same results up to the fp32 summation order.  Replaces the same decode fast path as
  * helm_int8_gemv (helm/kernels/fp16_gemv.cpp:105-157). */
 int64_t helm_int8_gemv_workspace_bytes(int M, int N, int K);
 /* Bytes with which helm_int8_gemv_ws takes its fastest form (0: no workspace
