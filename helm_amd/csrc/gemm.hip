@@ -406,12 +406,18 @@ Skinny pick_skinny(int M, int N, int K) {
   // start) against the partial sums' traffic (4 TB/s) and the second launch (3 us)
   const int nk = K / BK;
   const int64_t slots = 256 * skinny_occ(rt);
-  double best = -1.0;
+  double best = -1.0, whole = 0.0;
   for (int s = 1; s <= 32 && s <= std::max(1, nk / 4); ++s) {
     const double rounds = (double)((tiles * s + slots - 1) / slots);
     const double c = rounds * 0.4 * ((nk + s - 1) / s + 3) + (s > 1 ? 3.0 + (double)s * M * N * 8.0 / 4e6 : 0.0);
+    if (s == 1) whole = c;
     if (best < 0.0 || c < 0.97 * best) { best = c; p.s = s; }
   }
+  // full-height tiles on more than half of the CUs already: second workgroups on some
+  // CUs lengthen the chains there, so the price has to fall by an eighth (100 x 2560 -> 9728,
+  // 152 tiles, priced 6% less: 22.6 us in one slice, 24.3 in two; 100 x 4096 -> 12288,
+  // 192 tiles, 18% less: 33.5 and 30.2)
+  if (rt == 4 && tiles > 128 && tiles < 256 && best > 0.88 * whole) p.s = 1;
   // full-height tiles in one slice gain nothing over the prompt form's wider ones
   // (100 x 5120 -> 17408 58.8 against 57.8 us, 200 x 4096 -> 12288 43.3 against 42.5)
   if (rt == 4 && p.s == 1) p.rt = 0;

@@ -48,6 +48,17 @@ def test_gemm_tile_width_override(M, N, K, tn, monkeypatch, tmp_path):
     assert name.startswith(f"int8_gemm_kernel<{tn}, {'true' if tn >= 4 else 'false'}, 4, 3, false"), name
 
 
+@pytest.mark.parametrize("M,N,K,split", [(100, 9728, 2560, False), (97, 9728, 2560, False), (96, 9728, 2560, True),
+                                         (100, 12288, 4096, True), (100, 6144, 2560, True), (64, 4096, 4096, True)])
+def test_gemm_slices_by_price(M, N, K, split, tmp_path):
+    """The few-row form cuts K where that pays (its second pass adds the slices)."""
+    x = torch.randn(M, K, device="cuda").half()
+    q, s = int8_weights(N, K)
+    seen = launches(lambda: hk.int8_linear(x, q, s), tmp_path)
+    assert seen[0][0].startswith("int8_gemm_kernel<"), seen
+    assert [n.startswith("gemm_split_reduce_kernel") for n, _ in seen[1:]] == [True] * split, seen
+
+
 LDS, REGS, STREAM = "fp16_small_m_kernel<", "xreg_gemv_kernel<false", "gemv_stream_kernel<"
 
 
